@@ -503,7 +503,11 @@ struct zdx_sim {
         drop_graphs();
         if (rep) (void)hipHostFree(rep);
     }
+    // A step returns once its report is written, which is before the launch
+    // itself has retired: the graphs are destroyed only after the stream has
+    // drained.
     void drop_graphs() {
+        if (gexec[0] || gexec[1]) (void)hipStreamSynchronize(ctx->stream);
         for (int k = 0; k < 2; ++k) {
             if (gexec[k]) (void)hipGraphExecDestroy(gexec[k]);
             if (graph[k]) (void)hipGraphDestroy(graph[k]);
