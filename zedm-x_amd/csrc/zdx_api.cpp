@@ -210,6 +210,10 @@ struct zdx_ctx {
     DBuf<int32_t> m_voff, m_nv, m_toff, m_nt;
     DBuf<double> m_tol, m_aeps;
     DBuf<int32_t> m_soff, m_ns, m_susp;
+    DBuf<Cluster> m_clus;
+    DBuf<float> m_sph;
+    DBuf<int32_t> m_nc, m_coff, m_sphoff;
+    bool clusters = false;   // every mesh on the device has its clusters (else the hit-arena kernels run)
     // per-pair API buffers (api: grown with hipMalloc; api_na: carved from
     // na_arena, this device's no-allocation scratch, at every call)
     struct Api {
@@ -221,6 +225,8 @@ struct zdx_ctx {
         DBuf<int32_t> nondeg;
         DBuf<int32_t> pi, pj, order, npairs, status;
         DBuf<NarrowItem> items;
+        DBuf<PairItem> pitems;
+        DBuf<double> seg_tmp;
         DBuf<int64_t> seg_off, tri_checks, tri_tests;
         DBuf<int32_t> nseg, tri_hits, tri_scanned;
         DBuf<double> arena;
@@ -248,7 +254,7 @@ struct zdx_ctx {
         template <class F>
         void each_buf(F&& f) {
             f(pairs_in); f(mesh); f(state); f(wv_off); f(wt_off); f(wv); f(aabb); f(nondeg); f(pi); f(pj); f(order);
-            f(npairs); f(status); f(items); f(seg_off); f(tri_checks); f(tri_tests); f(nseg); f(tri_hits);
+            f(npairs); f(status); f(items); f(pitems); f(seg_tmp); f(seg_off); f(tri_checks); f(tri_tests); f(nseg); f(tri_hits);
             f(tri_scanned); f(arena); f(list_i); f(list_f); f(hits); f(hit_tri); f(hit_flag); f(hit_top); f(hit_off);
             f(queue); f(heavy); f(bcnt); f(bcur); f(ncontrib); f(comps); f(loops_raw); f(tstatus); f(topo_list); f(topo_n);
             f(status2); f(rec); f(vtx); f(prov); f(ej); f(vj); f(ljac); f(pk_loop_off); f(pk_seg_off);
@@ -278,6 +284,8 @@ struct zdx_ctx {
         M.verts = m_verts.p; M.tri_idx = m_tri.p; M.vert_off = m_voff.p; M.nverts = m_nv.p;
         M.tri_off = m_toff.p; M.ntris = m_nt.p; M.tol = m_tol.p; M.area_eps = m_aeps.p;
         M.susp_off = m_soff.p; M.nsusp = m_ns.p; M.susp = m_susp.p;
+        M.clusters = clusters ? m_clus.p : nullptr;
+        M.clus_sph = m_sph.p; M.nclus = m_nc.p; M.clus_off = m_coff.p; M.sph_off = m_sphoff.p;
         return M;
     }
     void sync_meshes() {
@@ -288,8 +296,23 @@ struct zdx_ctx {
         std::vector<int32_t> soff, ns, susp;
         // meshes with the same triangle indices (scaled copies of one shape)
         // share one copy on the device, so that the narrow phase's index
-        // loads stay in cache
-        std::unordered_map<uint64_t, std::vector<int32_t>> seen;   // hash -> first triangles of index arrays
+        // loads stay in cache.  So do a shape's clusters, and its vertices are
+        // numbered in their order on the device, so that a cluster's vertices
+        // lie together
+        struct Shape {
+            const std::vector<int32_t>* idx;
+            int32_t at, cl, ncl;         // its first triangle, its clusters
+            std::vector<int32_t> from;   // device vertex -> host vertex
+        };
+        std::unordered_map<uint64_t, std::vector<int32_t>> seen;   // hash -> shapes
+        std::vector<Shape> shapes;
+        std::vector<Cluster> cl;
+        std::vector<int32_t> nc, coff, sphoff;
+        int32_t nsph = 0;
+        clusters = true;
+        for (auto& m : meshes)
+            clusters = clusters && m.h.tri_idx.size() / 3 <= CLUSTER_MAX_TRIS &&
+                       m.h.verts.size() / 3 <= CLUSTER_MAX_VERTS;
         for (auto& m : meshes) {
             soff.push_back((int32_t)susp.size());
             ns.push_back((int32_t)m.h.suspect.size());
@@ -297,18 +320,38 @@ struct zdx_ctx {
             voff.push_back((int32_t)(v.size() / 3));
             nv.push_back((int32_t)(m.h.verts.size() / 3));
             nt.push_back((int32_t)(m.h.tri_idx.size() / 3));
-            v.insert(v.end(), m.h.verts.begin(), m.h.verts.end());
             uint64_t hsh = 1469598103934665603ull ^ m.h.tri_idx.size();
             for (int32_t x : m.h.tri_idx) hsh = (hsh ^ (uint32_t)x) * 1099511628211ull;
-            int32_t at = -1;
+            int32_t sh = -1;
             for (int32_t o : seen[hsh])
-                if (std::equal(m.h.tri_idx.begin(), m.h.tri_idx.end(), t.begin() + 3 * (size_t)o)) { at = o; break; }
-            if (at < 0) {
-                at = (int32_t)(t.size() / 3);
-                seen[hsh].push_back(at);
-                t.insert(t.end(), m.h.tri_idx.begin(), m.h.tri_idx.end());
+                if (*shapes[o].idx == m.h.tri_idx) { sh = o; break; }
+            if (sh < 0) {
+                sh = (int32_t)shapes.size();
+                seen[hsh].push_back(sh);
+                std::vector<Cluster> q;
+                if (clusters) q = cluster_mesh(m.h);
+                Shape s{&m.h.tri_idx, (int32_t)(t.size() / 3), (int32_t)cl.size(), (int32_t)q.size(), {}};
+                std::vector<int32_t> to(m.h.verts.size() / 3, -1);
+                auto number = [&](int32_t x) {
+                    if (to[x] < 0) {
+                        to[x] = (int32_t)s.from.size();
+                        s.from.push_back(x);
+                    }
+                    return to[x];
+                };
+                for (Cluster& k : q)
+                    for (uint16_t& x : k.v) x = (uint16_t)number(x);
+                for (int32_t x : m.h.tri_idx) t.push_back(number(x));
+                cl.insert(cl.end(), q.begin(), q.end());
+                shapes.push_back(std::move(s));
             }
-            toff.push_back(at);
+            for (int32_t x : shapes[sh].from)
+                v.insert(v.end(), m.h.verts.begin() + 3 * (size_t)x, m.h.verts.begin() + 3 * (size_t)x + 3);
+            nc.push_back(shapes[sh].ncl);
+            coff.push_back(shapes[sh].cl);
+            sphoff.push_back(nsph);
+            nsph += shapes[sh].ncl;
+            toff.push_back(shapes[sh].at);
             tol.push_back(m.tol);
             aeps.push_back(m.area_eps);
         }
@@ -323,6 +366,14 @@ struct zdx_ctx {
         m_soff.upload(soff.data(), soff.size(), stream);
         m_ns.upload(ns.data(), ns.size(), stream);
         m_susp.upload(susp.data(), susp.size(), stream);
+        if (clusters) {
+            m_clus.upload(cl.data(), cl.size(), stream);
+            m_nc.upload(nc.data(), nc.size(), stream);
+            m_coff.upload(coff.data(), coff.size(), stream);
+            m_sphoff.upload(sphoff.data(), sphoff.size(), stream);
+            m_sph.ensure(4 * (size_t)nsph);
+            launch_cluster_spheres(dmeshes(), (int32_t)meshes.size(), m_sph.p, stream);
+        }
         HIPC(hipStreamSynchronize(stream));
         mesh_dirty = false;
         ++mesh_version;
@@ -372,6 +423,8 @@ static __device__ __align__(256) unsigned char scratch[NOALLOC_SCRATCH_BYTES];
 // and the topology walks' scratch slices
 constexpr int64_t NOALLOC_LIST_BYTES = (int64_t)16 << 20;
 constexpr int64_t NOALLOC_WALK_SLICES = 256;
+// threads of the narrow phase's workgroups in the per-pair call
+constexpr int API_GROUP = 256;
 
 struct CallLimits {
     bool may_allocate = true;                       // false: device memory only from the arena
@@ -442,6 +495,8 @@ struct zdx_sim {
     } ps[2];
     DBuf<int32_t> d_order, d_bcnt, d_bcur, d_topo_list, d_topo_n, d_topo_big, d_topo_small, d_topo_nbs;
     DBuf<NarrowItem> d_items;
+    DBuf<PairItem> d_pitems;
+    DBuf<double> d_seg_tmp;
     DBuf<int64_t> d_seg_off, d_tri_checks, d_tri_tests;
     DBuf<int32_t> d_nseg, d_tri_hits, d_tri_scanned;
     DBuf<double> d_arena;        // segments, one slot per hit slot
@@ -548,6 +603,7 @@ struct zdx_sim {
         P.cap = pair_cap; P.n = ps[par].n.p; P.pi = ps[par].pi.p; P.pj = ps[par].pj.p;
         P.order = lpt ? d_order.p : nullptr;
         P.items = lpt ? d_items.p : nullptr;
+        P.pitems = d_pitems.p; P.seg_tmp = d_seg_tmp.p;
         P.seg_off = d_seg_off.p; P.nseg = d_nseg.p; P.tri_checks = d_tri_checks.p; P.tri_tests = d_tri_tests.p;
         P.tri_hits = d_tri_hits.p; P.tri_scanned = d_tri_scanned.p; P.arena = d_arena.p; P.arena_cap = hit_cap;
         P.status = d_status.p;
@@ -615,7 +671,7 @@ struct zdx_sim {
             HIPC(hipMemcpy(ps[k].n.p, &n, sizeof(int32_t), hipMemcpyHostToDevice));
         }
         d_adj_j.ensure(adj_cap); d_adj_pair.ensure(adj_cap);
-        d_order.ensure(cap); d_items.ensure(cap); d_heavy.ensure(cap); d_topo_list.ensure(cap); d_topo_n.ensure(1);
+        d_order.ensure(cap); d_items.ensure(cap); d_pitems.ensure(cap); d_heavy.ensure(cap); d_topo_list.ensure(cap); d_topo_n.ensure(1);
         d_topo_big.ensure(cap); d_topo_small.ensure(cap); d_topo_nbs.ensure(2);
         d_hit_off.ensure(cap); d_hit_top.ensure(HIT_SHARDS * HIT_TOP_STRIDE);
         d_seg_off.ensure(cap); d_tri_checks.ensure(cap); d_tri_tests.ensure(cap);
@@ -639,9 +695,24 @@ struct zdx_sim {
     void alloc_hits(int64_t cap) {
         drop_graphs();
         hit_cap = cap;
-        d_hits.release(); d_hit_flag.release(); d_arena.release();
-        d_hits.ensure(6 * (size_t)cap); d_hit_flag.ensure((size_t)cap); d_arena.ensure(6 * (size_t)cap);
+        d_hits.release(); d_hit_flag.release(); d_arena.release(); d_seg_tmp.release();
+        d_arena.ensure(6 * (size_t)cap);
         tw.ensure_arena(cap);
+        ensure_hits();
+    }
+    // the narrow phase's hits: 32 bytes each and their segments' place on the
+    // cluster path, 24 bytes on the hit-arena path, which also needs its
+    // workgroups' lists of kept triangles
+    void ensure_hits() {
+        d_hits.ensure((ctx->clusters ? 8 : 6) * (size_t)hit_cap);
+        d_hit_flag.ensure((size_t)hit_cap);
+        if (ctx->clusters) {
+            d_seg_tmp.ensure(6 * (size_t)hit_cap);
+            return;
+        }
+        const size_t groups = (size_t)std::max(1, ctx->n_cu * 16);
+        d_list_i.ensure(groups * 8 * (size_t)tmax);
+        d_list_f.ensure(groups * 12 * (size_t)tmax);
     }
     void alloc_topo_scratch() {
         drop_graphs();
@@ -715,10 +786,7 @@ void sim_setup_device(zdx_sim* s) {
         s->tw.adj_cap = 64; s->tw.snap_cap = 64; s->tw.tj_cap = 64; s->tw.units_cap = 4;
     }
     s->alloc_pairs(tiny ? 8 : std::max(1024, 8 * N));
-    size_t groups = (size_t)persistent_groups(c, 16);
     s->tmax = c->max_tris;
-    s->d_list_i.ensure(groups * 8 * (size_t)s->tmax);
-    s->d_list_f.ensure(groups * 12 * (size_t)s->tmax);
     s->topo_threads = std::min<int64_t>(2048, std::max<int64_t>(64, (int64_t)N));
     s->alloc_stage(s->stage_cap);
     s->alloc_hits(tiny ? 64 : std::max<int64_t>(1 << 16, 32 * (int64_t)N));
@@ -835,12 +903,14 @@ void enqueue_step(zdx_sim* s, int par, bool batched) {
     }
     int g_transform = s->transform_groups(), g_narrow = gmax, g_topo = (int)s->topo_threads,
         g_walls = (int)s->wall_threads;
+    int64_t n_pairs = 0;
     if (!batched) {
         int32_t c[3] = {0, 0, 0};
         HIPC(hipMemcpyAsync(&c[0], s->ps[par].n.p, 4, hipMemcpyDeviceToHost, st));
         HIPC(hipMemcpyAsync(&c[1], s->d_n_need.p, 4, hipMemcpyDeviceToHost, st));
         HIPC(hipMemcpyAsync(&c[2], s->d_n_wall.p, 4, hipMemcpyDeviceToHost, st));
         HIPC(hipStreamSynchronize(st));
+        n_pairs = c[0];
         g_narrow = std::max(1, std::min(c[0], gmax));
         g_transform = std::max(1, std::min(c[1], g_transform));
         g_walls = std::max(1, std::min(c[2], g_walls));
@@ -873,7 +943,13 @@ void enqueue_step(zdx_sim* s, int par, bool batched) {
     nc.use_queue = batched ? 1 : 0;
     nc.groups = g_narrow;
     nc.wave_groups = persistent_groups(s->ctx, 4);
-    launch_narrow(B, M, P, nc, s->d_list_i.p, s->d_list_f.p, s->stage_cap, s->tmax, s->d_queue.p, st, true, kt + 8);
+    nc.side = s->ctx->stream3; nc.ev_fork = s->ctx->ev_fork3; nc.ev_join = s->ctx->ev_join3;
+    // the pairs that bodies of like size can have (8 each, as the first
+    // pair buffers hold); plain mode has just read their number
+    nc.few = (batched ? std::min<int64_t>((int64_t)s->N * (s->N - 1) / 2, 8 * (int64_t)s->N) : n_pairs) <= PAIRS_FEW;
+    if (nc.few) nc.groups = (int)std::min<int64_t>(nc.groups, PAIRS_FEW);
+    launch_narrow(B, M, P, nc, s->d_list_i.p, s->d_list_f.p, s->stage_cap, s->tmax, s->d_queue.p, st,
+                  true, kt + 8);
     if (!batched) launch_stamp(kt + 3, st);   // batched: stamped by k_tp_alloc (no host read in between)
     if (!batched) {
         int32_t nt = 0;
@@ -986,6 +1062,7 @@ void step_once(zdx_sim* s, bool batched) {
     if (s->mesh_version != s->ctx->mesh_version) {
         s->drop_graphs();
         s->mesh_version = s->ctx->mesh_version;
+        s->ensure_hits();
     }
     for (int attempt = 0; attempt < 12; ++attempt) {
         const int par = s->parity;
@@ -1093,6 +1170,7 @@ void contact_pairs_impl(zdx_ctx* c, zdx_ctx::Api& A, const zdx_pair_in* pairs, i
         launch_transform(B, M, st);
         HIPC(hipEventRecord(c->ev_api[1], st));
         A.pi.ensure(n); A.pj.ensure(n); A.npairs.ensure(1); A.status.ensure(1); A.order.ensure(n); A.items.ensure(n);
+        A.pitems.ensure(n);
         A.status2.ensure(1);
         launch_iota_pairs(A.pi.p, A.pj.p, n, st);
         launch_fill_i32(A.npairs.p, n, 1, st);
@@ -1104,18 +1182,22 @@ void contact_pairs_impl(zdx_ctx* c, zdx_ctx::Api& A, const zdx_pair_in* pairs, i
         const bool batched = opts->mode == ZDX_MODE_BATCHED;
         int groups = std::min<int>(persistent_groups(c, 8), std::max(1, n));
         groups = (int)std::max<int64_t>(1, std::min<int64_t>(groups, lim.list_bytes / (80 * (int64_t)c->max_tris)));
-        A.list_i.ensure((size_t)groups * 8 * c->max_tris);
-        A.list_f.ensure((size_t)groups * 12 * c->max_tris);
+        if (!c->clusters) {
+            A.list_i.ensure((size_t)groups * 8 * c->max_tris);
+            A.list_f.ensure((size_t)groups * 12 * c->max_tris);
+        }
         const bool want_vtx = out->loop_vtx != nullptr;
         for (int attempt = 0; attempt < 10; ++attempt) {
             c->api_attempts = attempt + 1;
             A.arena.ensure((size_t)A.hit_cap * 6);
-            A.hits.ensure(6 * (size_t)A.hit_cap);
+            A.hits.ensure((c->clusters ? 8 : 6) * (size_t)A.hit_cap);
             A.hit_flag.ensure((size_t)A.hit_cap);
+            if (c->clusters) A.seg_tmp.ensure(6 * (size_t)A.hit_cap);
             const bool sens = opts->sensitivities != 0;
             DPairs P{};
             P.cap = n; P.n = A.npairs.p; P.pi = A.pi.p; P.pj = A.pj.p; P.order = batched ? A.order.p : nullptr;
             P.items = batched ? A.items.p : nullptr;
+            P.pitems = A.pitems.p; P.seg_tmp = A.seg_tmp.p;
             P.seg_off = A.seg_off.p; P.nseg = A.nseg.p; P.tri_checks = A.tri_checks.p; P.tri_tests = A.tri_tests.p;
             P.tri_hits = A.tri_hits.p; P.tri_scanned = A.tri_scanned.p; P.arena = A.arena.p; P.arena_cap = A.hit_cap;
             P.status = A.status.p;
@@ -1134,7 +1216,9 @@ void contact_pairs_impl(zdx_ctx* c, zdx_ctx::Api& A, const zdx_pair_in* pairs, i
             launch_fill_i32(A.topo_n.p, 0, 1, st);
             HIPC(hipEventRecord(c->ev_api[2], st));
             if (batched) launch_lpt_order(P, M, B, A.order.p, A.bcnt.p, A.bcur.p, n, st);
-            NarrowCfg nc{256, 4, groups, batched ? 1 : 0, std::min(persistent_groups(c, 4), (n + 3) / 4)};
+            NarrowCfg nc{API_GROUP, 4, groups, batched ? 1 : 0, std::min(persistent_groups(c, 4), (n + 3) / 4)};
+            nc.side = c->stream3; nc.ev_fork = c->ev_fork3; nc.ev_join = c->ev_join3;
+            nc.few = n <= PAIRS_FEW;
             launch_narrow(B, M, P, nc, A.list_i.p, A.list_f.p, A.stage_cap, c->max_tris, A.queue.p, st);
             HIPC(hipEventRecord(c->ev_api[3], st));
             int32_t status = 0;
@@ -1800,6 +1884,7 @@ zdx_status zdx_sim_autotune(zdx_sim* s, int32_t* out_block, int32_t* out_groups)
     return guard(s->ctx, [&] {
         hipStream_t st = s->st();
         const int par = s->parity;
+        s->ensure_hits();
         DBodies B = s->bodies(par);
         DMeshes M = s->ctx->dmeshes();
         launch_fill_i32(s->d_status.p, 0, 1, st);
@@ -1830,13 +1915,14 @@ zdx_status zdx_sim_autotune(zdx_sim* s, int32_t* out_block, int32_t* out_groups)
         for (auto& cb : cand) {
             for (int g : gpc) for (int wt : wtests) {
                 NarrowCfg nc{cb[0], cb[1], persistent_groups(s->ctx, g), 1, persistent_groups(s->ctx, 4), wt};
+                nc.side = s->ctx->stream3; nc.ev_fork = s->ctx->ev_fork3; nc.ev_join = s->ctx->ev_join3;
                 // one untimed launch, then the median of four timed ones
                 float t4[4] = {0, 0, 0, 0};
                 for (int rep = 0; rep < 5; ++rep) {
                     launch_fill_i32(s->d_topo_n.p, 0, 1, st);
                     HIPC(hipEventRecord(e0, st));
-                    launch_narrow(B, M, P, nc, s->d_list_i.p, s->d_list_f.p, s->stage_cap, s->tmax, s->d_queue.p,
-                                  st);
+                    launch_narrow(B, M, P, nc, s->d_list_i.p, s->d_list_f.p, s->stage_cap, s->tmax,
+                                  s->d_queue.p, st);
                     HIPC(hipEventRecord(e1, st));
                     HIPC(hipEventSynchronize(e1));
                     float ms = 0;

@@ -2,6 +2,7 @@
 // parsing and particle constants, restating src/main.cpp of
 // zhl-handsome/ZEDM-X (lines cited per function) with the same FP64
 // operation order (the library is built with -ffp-contract=off).
+#include <algorithm>
 #include <cctype>
 #include <cmath>
 #include <cstring>
@@ -247,6 +248,74 @@ HostMesh build_mesh(const std::vector<double>& in, bool center) {
         }
     }
     return m;
+}
+
+std::vector<Cluster> cluster_mesh(const HostMesh& m) {
+    std::vector<Cluster> out;
+    const int32_t T = (int32_t)(m.tri_idx.size() / 3);
+    if ((size_t)T > CLUSTER_MAX_TRIS || m.verts.size() / 3 > CLUSTER_MAX_VERTS) return out;
+    struct Tri { double c[3]; int32_t t; };
+    std::vector<Tri> o((size_t)T);
+    const double* v = m.verts.data();
+    for (int32_t t = 0; t < T; ++t) {
+        const int32_t* ix = &m.tri_idx[3 * (size_t)t];
+        o[t].t = t;
+        for (int k = 0; k < 3; ++k) {
+            const double x = v[3 * (size_t)ix[0] + k] + v[3 * (size_t)ix[1] + k] + v[3 * (size_t)ix[2] + k];
+            o[t].c[k] = std::isfinite(x) ? x : 0.0;   // a strict order for nth_element
+        }
+    }
+    // the triangles o[b..e) into as few clusters as their corners allow
+    auto emit = [&](int32_t b, int32_t e) {
+        while (b < e) {
+            Cluster q;
+            int nv = 0, nt = 0;
+            for (; b < e && nt < CT; ++b) {
+                const int32_t* ix = &m.tri_idx[3 * (size_t)o[b].t];
+                uint32_t w = 0;
+                int n = nv;
+                for (int k = 0; k < 3 && n <= CT; ++k) {
+                    int l = 0;
+                    while (l < n && q.v[l] != (uint16_t)ix[k]) ++l;
+                    if (l == n && n < CT) q.v[n] = (uint16_t)ix[k];
+                    if (l == n) ++n;   // CT + 1: the triangle does not fit
+                    w |= (uint32_t)(l & 15) << (4 * k);
+                }
+                if (n > CT) break;
+                nv = n;
+                q.t[nt++] = w | (uint32_t)o[b].t << 16;
+            }
+            for (int l = nv; l < CT; ++l) q.v[l] = q.v[0];
+            for (int k = nt; k < CT; ++k) q.t[k] = CLUS_NONE << 16;
+            out.push_back(q);
+        }
+    };
+    std::vector<std::pair<int32_t, int32_t>> todo{{0, T}};
+    while (!todo.empty()) {
+        const auto [b, e] = todo.back();
+        todo.pop_back();
+        if (e - b <= CT) {
+            emit(b, e);
+            continue;
+        }
+        double lo[3], hi[3];
+        for (int k = 0; k < 3; ++k) lo[k] = hi[k] = o[b].c[k];
+        for (int32_t q = b + 1; q < e; ++q)
+            for (int k = 0; k < 3; ++k) {
+                lo[k] = o[q].c[k] < lo[k] ? o[q].c[k] : lo[k];
+                hi[k] = o[q].c[k] > hi[k] ? o[q].c[k] : hi[k];
+            }
+        int ax = 0;
+        for (int k = 1; k < 3; ++k)
+            if (hi[k] - lo[k] > hi[ax] - lo[ax]) ax = k;
+        const int32_t half = std::max(CT, ((e - b) / 2 + CT / 2) / CT * CT);
+        std::nth_element(o.begin() + b, o.begin() + b + half, o.begin() + e, [&](const Tri& x, const Tri& y) {
+            return x.c[ax] < y.c[ax] || (x.c[ax] == y.c[ax] && x.t < y.t);
+        });
+        todo.push_back({b + half, e});
+        todo.push_back({b, b + half});
+    }
+    return out;
 }
 
 // parse_config_file, src/main.cpp:1531-1689

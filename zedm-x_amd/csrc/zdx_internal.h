@@ -119,7 +119,26 @@ ParticleConst particle_const(const HostMesh& m, int mesh_id, double density, dou
 // L = I_world * omega (src/main.cpp:1985)
 void initial_L(const ParticleConst& c, const double* quat, const double* omega, double* L);
 
+// A cluster: a compact patch of at most CT triangles with at most CT corners
+// between them.  v: its vertices (unused entries repeat the first); t: per
+// triangle its corners as indices into v, 4 bits each, and from bit 16 on its
+// index in the mesh (CLUS_NONE: no triangle).
+constexpr int CT = 16;
+constexpr uint32_t CLUS_NONE = 0xffffu;
+struct Cluster {
+    uint16_t v[CT];
+    uint32_t t[CT];
+};
+// The mesh's triangles in clusters (k-d splits of their centroids), every
+// triangle once; empty when the mesh exceeds the 16-bit indices.
+constexpr size_t CLUSTER_MAX_TRIS = 65535, CLUSTER_MAX_VERTS = 65536;
+std::vector<Cluster> cluster_mesh(const HostMesh& m);
+
 // ---------------------------------------------------------------- device views
+// A kept triangle of the narrow phase: its corners (mesh-local vertices) and
+// its index in the mesh.
+struct alignas(8) TriQ { uint16_t a, b, c, id; };
+
 // Registered meshes, concatenated.
 struct DMeshes {
     const double* verts;     // body-frame vertices
@@ -133,6 +152,15 @@ struct DMeshes {
     const int32_t* susp_off; // per mesh: first suspect triangle in susp
     const int32_t* nsusp;    // per mesh: triangles whose world plane may degenerate
     const int32_t* susp;     // suspect triangle indices
+    // clusters of each mesh's triangles (shared by meshes with the same
+    // triangle indices) and their bounding spheres in the body frame (x, y, z,
+    // radius); clusters is nullptr when a registered mesh exceeds the 16-bit
+    // indices
+    const Cluster* clusters;
+    const float* clus_sph;
+    const int32_t* nclus;    // per mesh
+    const int32_t* clus_off; // per mesh: first cluster
+    const int32_t* sph_off;  // per mesh: first sphere
 };
 
 // Bodies whose world geometry is evaluated each step.
@@ -169,6 +197,21 @@ struct NarrowItem {
     float boxA[6], boxB[6];
     int32_t pad[8];
 };
+// One pair of the cluster kernels in work order (make_pair_item); index 0 is A,
+// 1 is B.
+struct PairItem {
+    int32_t p, nondegA, T[2], wo[2], nc[2], co[2], so[2];   // triangles, first world vertex, clusters: count,
+                                                            // first cluster, first sphere
+    float R[2][9], t[2][3], H[2][3], th[2][6];
+    int32_t pad[10];
+};
+// One hit of the cluster kernels: the six world-vertex indices, (ta << 16) | tb
+// and the pair.
+struct PairHit {
+    int32_t v[6];
+    uint32_t key;
+    int32_t pair;
+};
 
 // The hit arena is cut into shards, each with its own counter: a pair's
 // hits go to shard (work item % hit_shards), so that the reservations are
@@ -185,6 +228,8 @@ struct DPairs {
     const int32_t* pj;       // body B
     const int32_t* order;    // processing order (LPT in batched mode)
     NarrowItem* items;       // with order: the pairs' narrow-phase items in that order
+    PairItem* pitems;        // with clusters: their items, in that order (else in pair order)
+    double* seg_tmp;         // with clusters: segments before they are put in order, 6 doubles per hit slot
     int64_t* seg_off;        // per pair: first segment in the arena
     int32_t* nseg;           // per pair
     int64_t* tri_checks;     // per pair (reference counter)

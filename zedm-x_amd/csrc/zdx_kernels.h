@@ -139,7 +139,17 @@ struct NarrowCfg {
     int32_t use_queue;         // 1: atomic work queue (batched)
     int32_t wave_groups;       // workgroups of the one-wave-per-pair kernel (0: 4 per CU's worth of groups)
     int32_t wave_tests;        // most float-box tests of a pair on the one-wave kernel (0: its default)
+    // cluster path: the workgroups of the pairs below the largest run on
+    // `side`, forked from and joined back into the launch's stream (nullptr: in
+    // a row)
+    hipStream_t side = nullptr;
+    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+    // cluster path: few pairs (PAIRS_FEW), each by a workgroup at once
+    bool few = false;
 };
+// The most pairs that get a workgroup each at once: two workgroups of 512
+// threads fit on each of 256 CUs.
+constexpr int64_t PAIRS_FEW = 512;
 
 // Writes the device clock into *slot when the stream reaches it (NULL: no-op).
 void launch_stamp(unsigned long long* slot, hipStream_t s);
@@ -197,12 +207,17 @@ void launch_broadphase(const BroadPhaseBufs& bp, hipStream_t s, const NeedLists*
 // pair may store (ST_STAGE beyond); queue: the cull's work counter; resets
 // the queue and P.hit_top itself unless the caller did (zeroed).
 // queue: NARROW_COUNTERS counters (the wave kernel's work queues, the heavy
-// list's front and back counts, the workgroup kernel's queue over it, each on a
-// 128-byte line of its own), zeroed here unless `zeroed`.
-constexpr int NARROW_COUNTERS = 67 * 32;
+// list's front and back counts, the workgroup kernels' queues over it, each on
+// a 128-byte line of its own), zeroed here unless `zeroed`.
+constexpr int NARROW_COUNTERS = 68 * 32;
+// With clusters (M.clusters) the kernels of zdx_cluster.h, which use neither
+// list_i nor list_f, else those of zdx_narrow.h.
 void launch_narrow(const DBodies& B, const DMeshes& M, const DPairs& P, const NarrowCfg& cfg, int32_t* list_i,
                    float* list_f, int32_t seg_cap, int32_t tmax, unsigned int* queue, hipStream_t s, bool zeroed = false,
                    unsigned long long* stamp = nullptr);
+// Bounding spheres of the clusters of n meshes into sph (4 floats each, at
+// M.sph_off).
+void launch_cluster_spheres(const DMeshes& M, int32_t n, float* sph, hipStream_t s);
 // LPT work order of the pairs (largest estimated cost first) into order,
 // and the narrow-phase items (P.items, when set) in that order; zeroed:
 // bucket_cnt and bucket_cur (64 each) already hold 0

@@ -766,6 +766,7 @@ __device__ long long g_snap_hits[8192];
 // ------------------------------------------------------------ narrow phase
 #include "zdx_narrow.h"
 static_assert(NQ_COUNTERS == NARROW_COUNTERS, "narrow-phase counters");
+#include "zdx_cluster.h"
 
 // Narrow phase, part 2 (exact tests): one thread per hit of the hit arena.
 // Each hit is re-tested with the reference's exact AABB reject
@@ -838,10 +839,6 @@ __global__ void __launch_bounds__(256) k_narrow_exact(DBodies B, DPairs P) {
         }
     }
 }
-
-// pairs with at least this many segments are walked first (their walks are
-// the longest, so they should not wait for a free workgroup)
-constexpr int TOPO_BIG_SEGS = 40;
 
 // Narrow phase, part 3: one wave per pair compacts its segments in hit
 // order, i.e. in the reference's (ta, tb) order, to the front of its hit
@@ -974,8 +971,34 @@ __global__ void __launch_bounds__(256) k_lpt_count(DPairs P, DMeshes M, DBodies 
     __syncthreads();
     if (threadIdx.x < 64 && h[threadIdx.x]) atomicAdd(&bucket_cnt[threadIdx.x], h[threadIdx.x]);
 }
+// Work item of pair p at `slot`.
+__device__ inline void make_item(const DPairs& P, const DMeshes& M, const DBodies& B, int p, int slot) {
+    if (M.clusters) {
+        PairItem o;
+        make_pair_item(P, M, B, p, o);
+        P.pitems[slot] = o;
+        return;
+    }
+    NarrowItem it;
+    const int i = P.pi[p], j = P.pj[p];
+    const int mA = B.mesh[i], mB = B.mesh[j];
+    it.p = p; it.i = i; it.j = j;
+    it.TA = M.ntris[mA]; it.TB = M.ntris[mB];
+    it.VA = M.nverts[mA]; it.VB = M.nverts[mB];
+    it.toA = M.tri_off[mA]; it.toB = M.tri_off[mB];
+    it.woA = (int32_t)B.wv_off[i]; it.woB = (int32_t)B.wv_off[j];
+    it.nondegA = B.nondeg[i];
+    box_f(B.aabb + 6 * (int64_t)i, B.aabb + 6 * (int64_t)i + 3, it.boxA);
+    box_f(B.aabb + 6 * (int64_t)j, B.aabb + 6 * (int64_t)j + 3, it.boxB);
+    for (int k = 0; k < 8; ++k) it.pad[k] = 0;
+    P.items[slot] = it;
+}
+// the items in pair order (no work ordering)
+__global__ void __launch_bounds__(256) k_pair_items(DPairs P, DMeshes M, DBodies B) {
+    const int n = *P.n;
+    for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x) make_item(P, M, B, p, p);
+}
 // order within a bucket is free (any order gives the same per-pair results)
-__device__ inline void box_f(const double* lo, const double* hi, float* f);
 __global__ void __launch_bounds__(256) k_lpt_scatter(DPairs P, DMeshes M, DBodies B, const int32_t* bucket_cnt,
                                                      int32_t* bucket_cur, int32_t* order, TopoBufs T,
                                                      uint8_t* cur_active, int32_t tz) {
@@ -1017,21 +1040,7 @@ __global__ void __launch_bounds__(256) k_lpt_scatter(DPairs P, DMeshes M, DBodie
             }
             const int slot = base[b] + r;
             order[slot] = p;
-            if (P.items) {
-                NarrowItem it;
-                const int i = P.pi[p], j = P.pj[p];
-                const int mA = B.mesh[i], mB = B.mesh[j];
-                it.p = p; it.i = i; it.j = j;
-                it.TA = M.ntris[mA]; it.TB = M.ntris[mB];
-                it.VA = M.nverts[mA]; it.VB = M.nverts[mB];
-                it.toA = M.tri_off[mA]; it.toB = M.tri_off[mB];
-                it.woA = (int32_t)B.wv_off[i]; it.woB = (int32_t)B.wv_off[j];
-                it.nondegA = B.nondeg[i];
-                box_f(B.aabb + 6 * (int64_t)i, B.aabb + 6 * (int64_t)i + 3, it.boxA);
-                box_f(B.aabb + 6 * (int64_t)j, B.aabb + 6 * (int64_t)j + 3, it.boxB);
-                for (int k = 0; k < 8; ++k) it.pad[k] = 0;
-                P.items[slot] = it;
-            }
+            make_item(P, M, B, p, slot);
         }
         __syncthreads();
     }
@@ -2292,6 +2301,67 @@ static void narrow_t(const DBodies& B, const DMeshes& M, const DPairs& P, const 
                        lf, tmax, cfg.use_queue, q + NQ_WG, P.heavy, q + NQ_HEAVY, q + NQ_HEAVY_BACK, nullptr);
 }
 
+// the cluster path
+static void launch_pairs(const DBodies& B, const DMeshes& M, const DPairs& P, const NarrowCfg& cfg, int32_t seg_cap,
+                         unsigned int* q, hipStream_t s, int wave_groups, int32_t wave_tests,
+                         unsigned long long* stamp) {
+    // without the work ordering (plain mode) the items in pair order
+    if (!P.order)
+        hipLaunchKernelGGL(k_pair_items, dim3(std::max(1, std::min(nblk(P.cap, 256), 1024))), dim3(256), 0, s, P, M, B);
+    auto group = [&](auto kernel, int bs, int back, hipStream_t gs) {
+        const int32_t* count = back < 0 ? P.n : (const int32_t*)(q + (back ? NQ_HEAVY_BACK : NQ_HEAVY));
+        hipLaunchKernelGGL(kernel, dim3(cfg.groups), dim3(bs), (size_t)pairs_group_lds_bytes(bs), gs, B, M, P,
+                           cfg.use_queue, q + (back > 0 ? NQ_WG : NQ_WG_FRONT),
+                           back < 0 ? (const int32_t*)nullptr : (const int32_t*)P.heavy, count, back,
+                           back < 0 ? stamp : nullptr);
+    };
+    const int ge = std::max(1, cfg.groups) * 4;   // grid-stride over the hits
+    const int gs = std::max(1, std::min(nblk(P.cap, 4), 1024));
+    auto finish = [&] {
+        if (P.prov) {
+            hipLaunchKernelGGL(k_pairs_exact<true>, dim3(ge), dim3(256), 0, s, B, P);
+            hipLaunchKernelGGL(k_pairs_sort<true>, dim3(gs), dim3(256), 0, s, P, seg_cap);
+        } else {
+            hipLaunchKernelGGL(k_pairs_exact<false>, dim3(ge), dim3(256), 0, s, B, P);
+            hipLaunchKernelGGL(k_pairs_sort<false>, dim3(gs), dim3(256), 0, s, P, seg_cap);
+        }
+    };
+    // a workgroup for every pair: no wave kernel before it, no second list, no
+    // fork
+    if (cfg.few) {
+        group(k_pairs_group<GROUP_BIG>, GROUP_BIG, -1, s);
+        finish();
+        return;
+    }
+    hipLaunchKernelGGL(k_pairs_wave, dim3(wave_groups), dim3(NWV * WAVE), (size_t)pairs_wave_lds_bytes(), s, B, M, P,
+                       P.heavy, q, cfg.use_queue, wave_tests, stamp);
+    // the two lists side by side (in a row each launch lasts as long as its
+    // slowest pair, 40 to 60 us), the larger pairs on this stream: they start at
+    // once, before the others take the CUs' LDS
+    const bool fork = cfg.side && cfg.ev_fork && cfg.ev_join;
+    if (fork) {
+        (void)hipEventRecord(cfg.ev_fork, s);
+        (void)hipStreamWaitEvent(cfg.side, cfg.ev_fork, 0);
+    }
+    group(k_pairs_group<GROUP_BIG>, GROUP_BIG, 0, s);
+    hipStream_t sb = fork ? cfg.side : s;
+    switch (cfg.block) {
+        case 64: group(k_pairs_group<64>, 64, 1, sb); break;
+        case 128: group(k_pairs_group<128>, 128, 1, sb); break;
+        case 512: group(k_pairs_group<512>, 512, 1, sb); break;
+        default: group(k_pairs_group<256>, 256, 1, sb); break;
+    }
+    if (fork) {
+        (void)hipEventRecord(cfg.ev_join, cfg.side);
+        (void)hipStreamWaitEvent(s, cfg.ev_join, 0);
+    }
+    finish();
+}
+
+void launch_cluster_spheres(const DMeshes& M, int32_t n, float* sph, hipStream_t s) {
+    if (n > 0) hipLaunchKernelGGL(k_cluster_spheres, dim3(n), dim3(256), 0, s, M, sph);
+}
+
 void launch_narrow(const DBodies& B, const DMeshes& M, const DPairs& P, const NarrowCfg& cfg, int32_t* li, float* lf,
                    int32_t seg_cap, int32_t tmax, unsigned int* q, hipStream_t s, bool zeroed,
                    unsigned long long* stamp) {
@@ -2302,7 +2372,11 @@ void launch_narrow(const DBodies& B, const DMeshes& M, const DPairs& P, const Na
     // every pair through the one-wave kernel; the pairs it leaves (heavy)
     // through the workgroup kernel of the configured shape
     const int wg = cfg.wave_groups > 0 ? cfg.wave_groups : std::max(1, cfg.groups);
-    const int32_t wt = cfg.wave_tests > 0 ? cfg.wave_tests : (int32_t)W_HEAVY_TESTS;
+    const int32_t wt = cfg.wave_tests > 0 ? cfg.wave_tests : (int32_t)(M.clusters ? CW_TESTS : W_HEAVY_TESTS);
+    if (M.clusters) {
+        launch_pairs(B, M, P, cfg, seg_cap, q, s, wg, wt, stamp);
+        return;
+    }
     hipLaunchKernelGGL(k_narrow_wave<4>, dim3(wg), dim3(NWV * WAVE), (size_t)narrow_wave_lds_bytes(), s, B, M, P,
                        P.heavy, q, cfg.use_queue, wt, stamp);
     const int key = P.prov ? 25604 : cfg.block * 100 + cfg.items;

@@ -613,11 +613,11 @@ constexpr int NWV = 4;
 constexpr int WSLICE = 9728;
 // the narrow phase's counters (zeroed before it), each on a 128-byte line of
 // its own (atomics on one line serialise): WQ work queues of the wave kernel,
-// then the heavy list's two counts (front, back) and the workgroup kernel's queue
+// then the heavy list's two counts (front, back) and the workgroup kernels' queues
 constexpr int WQ = 64;
 constexpr int QSTRIDE = 32;   // in 4-byte counters
 constexpr int NQ_HEAVY = WQ * QSTRIDE, NQ_WG = (WQ + 1) * QSTRIDE, NQ_HEAVY_BACK = (WQ + 2) * QSTRIDE,
-              NQ_COUNTERS = (WQ + 3) * QSTRIDE;
+              NQ_WG_FRONT = (WQ + 3) * QSTRIDE, NQ_COUNTERS = (WQ + 4) * QSTRIDE;
 // heavy pairs of at least this many float-box tests (or too many vertices for
 // the wave) go to the front of the heavy list, the others to its back, so that
 // the workgroup kernel starts the costliest first
