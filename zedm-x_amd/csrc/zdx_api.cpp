@@ -947,7 +947,13 @@ void enqueue_step(zdx_sim* s, int par, bool batched) {
     // the pairs that bodies of like size can have (8 each, as the first
     // pair buffers hold); plain mode has just read their number
     nc.few = (batched ? std::min<int64_t>((int64_t)s->N * (s->N - 1) / 2, 8 * (int64_t)s->N) : n_pairs) <= PAIRS_FEW;
-    if (nc.few) nc.groups = (int)std::min<int64_t>(nc.groups, PAIRS_FEW);
+    if (nc.few) {
+        nc.groups = (int)std::min<int64_t>(nc.groups, PAIRS_FEW);
+        // one launch per topology stage, and two walks per CU at most: no big
+        // list beside the others, more LDS each
+        P.topo_big = P.topo_small = P.n_big = P.n_small = nullptr;
+        T.lds_bytes = std::max(T.lds_bytes, TOPO_LDS_FEW);
+    }
     launch_narrow(B, M, P, nc, s->d_list_i.p, s->d_list_f.p, s->stage_cap, s->tmax, s->d_queue.p, st,
                   true, kt + 8);
     if (!batched) launch_stamp(kt + 3, st);   // batched: stamped by k_tp_alloc (no host read in between)
@@ -1236,7 +1242,7 @@ void contact_pairs_impl(zdx_ctx* c, zdx_ctx::Api& A, const zdx_pair_in* pairs, i
             T.nthreads = std::min<int64_t>(lim.walk_slices, (int64_t)n);
             T.pass_groups = std::min<int64_t>(2048, (int64_t)n);
             T.seg_max = A.stage_cap;
-            T.lds_bytes = 32 * 1024;
+            T.lds_bytes = nc.few ? TOPO_LDS_FEW : 32 * 1024;
             T.vmax = 4 * A.stage_cap + 16;
             T.k_stiff = opts->k;
             T.tol_override = opts->tol > 0.0 ? opts->tol : 0.0;

@@ -150,6 +150,8 @@ struct NarrowCfg {
 // The most pairs that get a workgroup each at once: two workgroups of 512
 // threads fit on each of 256 CUs.
 constexpr int64_t PAIRS_FEW = 512;
+// LDS of a topology walk then (two per CU).
+constexpr int32_t TOPO_LDS_FEW = 76 * 1024;
 
 // Writes the device clock into *slot when the stream reaches it (NULL: no-op).
 void launch_stamp(unsigned long long* slot, hipStream_t s);

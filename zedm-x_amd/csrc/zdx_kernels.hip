@@ -1151,30 +1151,7 @@ struct LaneDev {
 // (persistent); walk kernels: one wave per pair, scratch in LDS when it fits,
 // else the workgroup's slice of the global scratch.
 
-// Snap / adjacency tolerance of a pair: mesh A's (main.cpp:2118-2121) unless
-// the caller of the per-pair API gave one.
-__device__ inline double topo_tol(const TopoBufs& T, const DMeshes& M, int mesh_a) {
-    return T.tol_override > 0.0 ? T.tol_override : M.tol[mesh_a];
-}
-
-constexpr int TP_PASS_A_SEGS = 384;     // segments pass A stages in LDS (84 bytes each)
-constexpr int TP_PASS_A_KEYS = 8192;    // LDS bytes for a unit's rows x S key matrix
-constexpr int TP_PASS_A_WORDS = 256;    // snap words a unit builds in LDS at a time
-constexpr int TP_PASS_A_THREADS = 1024;
-constexpr int TP_PASS_A_TESTS = 4096;   // segment-pair tests per unit (sets the units of a big pair)
-
-// Units of pass A for a pair of S segments: enough that each unit has at most
-// TP_PASS_A_TESTS candidate tests (rows x S) and TP_PASS_A_WORDS snap words,
-// and at least one row.
-__device__ inline int tp_pa_units(int S) {
-    const int64_t npt = (int64_t)S * (2 * S - 1);
-    const int64_t nw = (npt + 63) >> 6;
-    int64_t m = ((int64_t)S * S + TP_PASS_A_TESTS - 1) / TP_PASS_A_TESTS;
-    const int64_t mw = (nw + TP_PASS_A_WORDS - 1) / TP_PASS_A_WORDS;
-    if (mw > m) m = mw;
-    if (m > S) m = S;
-    return m < 1 ? 1 : (int)m;
-}
+#include "zdx_pass_a.h"
 
 // Pass A allocation, one thread per work-list item: the item's adjacency rows
 // and snap words (bump counters top[0], top[1]) and, for a pair split into
@@ -1203,127 +1180,6 @@ __global__ void __launch_bounds__(256) k_tp_alloc(DPairs P, TopoBufs T) {
         }
         T.adj_off[it] = ok ? ao : -1;
         T.snap_off[it] = ok ? so : -1;
-    }
-}
-
-// Pass A: representative-point cells, the adjacency rows (per segment the
-// count and up to R accepted candidates in ascending j) and the snap hit words
-// of every pair.  One 1024-thread workgroup per unit: unit 0 of every item,
-// then the extra units of the big pairs.  A unit of a pair split into nu
-// units takes a band of rows and a range of snap words of its own.  The
-// segments and cells are staged in LDS; the candidate tests of the band run
-// flat into an LDS key matrix that one thread per row then compacts; the snap
-// words are built in LDS (each thread a contiguous range of endpoint pairs)
-// and stored whole.
-// MODE 0: every item and every extra unit; MODE 1: the items of
-// P.topo_small only (fewer than TOPO_BIG_SEGS segments, so one unit each);
-// MODE 2: the items of P.topo_big and every extra unit.  KEYS and WORDS size
-// the LDS key matrix and snap-word chunk.
-template <int NT_MAX, int KEYS, int WORDS, int MODE>
-__global__ void __launch_bounds__(NT_MAX) k_tp_pass_a(DPairs P, DMeshes M, DBodies B, TopoBufs T,
-                                                     int32_t lds_segs) {
-    extern __shared__ char s_pa[];
-    const int n = MODE == 0 ? *P.topo_n : (MODE == 1 ? *P.n_small : *P.n_big);
-    const int nunits = n + (MODE == 1 ? 0 : (int)*(T.top + 4));
-    const int R = T.adj_row;
-    const int NT = blockDim.x;
-    uint8_t* keys = (uint8_t*)(s_pa + 84 * (int64_t)lds_segs);
-    unsigned long long* sw = (unsigned long long*)(s_pa + 84 * (int64_t)lds_segs + KEYS);
-    for (int u = blockIdx.x; u < nunits; u += gridDim.x) {
-#ifdef ZDX_WALK_PROFILE
-        const unsigned long long pa_t0 = wall_clock64();
-#endif
-        int it = MODE == 0 ? u : (u < n ? (MODE == 1 ? P.topo_small[u] : P.topo_big[u]) : 0), b = 0;
-        if (u >= n) {
-            if (u - n >= T.units_cap) continue;
-            const int2 e = ((const int2*)T.units)[u - n];
-            it = e.x;
-            b = e.y;
-            // k_tp_alloc wrote every slot below units_cap this step; this only
-            // guards against a slot it did not write
-            if (it < 0 || it >= *P.topo_n || b < 1) continue;
-        }
-        const long long ao = T.adj_off[it], so = T.snap_off[it];
-        if (ao < 0) continue;
-        const int p = P.topo_list[it];
-        const int S = P.nseg[p];
-        if (b >= tp_pa_units(S)) continue;
-        const int64_t sb = P.seg_off[p];
-        const double h = topo_tol(T, M, B.mesh[P.pi[p]]);
-        const double* gseg = P.arena + 6 * sb;
-        int* gc9 = T.cell9 + 9 * sb;
-        const bool staged = S <= lds_segs;
-        double* seg = staged ? (double*)s_pa : (double*)gseg;
-        int* c9 = staged ? (int*)(s_pa + 48 * (int64_t)lds_segs) : gc9;
-        const int nu = tp_pa_units(S);
-        const int r0 = (int)((int64_t)b * S / nu), r1 = (int)((int64_t)(b + 1) * S / nu);
-        const int npt = S * (2 * S - 1);   // endpoint pairs of 2S points
-        const int nw = (npt + 63) >> 6;
-        const int w0 = (int)((int64_t)b * nw / nu), w1 = (int)((int64_t)(b + 1) * nw / nu);
-        if (staged)
-            for (int k = threadIdx.x; k < 6 * S; k += NT) seg[k] = gseg[k];
-        __syncthreads();
-        for (int k = threadIdx.x; k < S; k += NT) tp_cells(seg, k, h, c9 + 9 * k);
-        __syncthreads();
-        int* cntp = T.adj + ao;
-        int* rows = cntp + S;
-        const int nr = r1 - r0;
-        if (nr * S <= KEYS) {
-            for (int k = threadIdx.x; k < nr * S; k += NT) {
-                const int i = r0 + k / S, j = k - (k / S) * S;
-                keys[k] = (uint8_t)tp_adj_key(seg, c9, h, i, j);
-            }
-            __syncthreads();
-            for (int i = r0 + (int)threadIdx.x; i < r1; i += NT) {
-                const uint8_t* kr = keys + (i - r0) * S;
-                int* out = rows + (int64_t)i * R;
-                int m = 0;
-                for (int j = 0; j < S; ++j) {
-                    const int key = kr[j];
-                    if (key == TP_NOADJ) continue;
-                    if (m < R) out[m] = j | (key << 24);
-                    ++m;
-                }
-                cntp[i] = m;
-                if (m > R) atomicMax(T.top + 3, (unsigned long long)m);
-            }
-        } else {
-            for (int i = r0 + (int)threadIdx.x; i < r1; i += NT) {
-                const int m = tp_adj_row(seg, c9, h, S, i, rows + (int64_t)i * R, R);
-                cntp[i] = m;
-                if (m > R) atomicMax(T.top + 3, (unsigned long long)m);
-            }
-        }
-        // snap hits of the unit's words, WORDS at a time: each
-        // thread a contiguous range of pair numbers t (a(a-1)/2 + b) sets bits
-        // in LDS, then the words are stored whole
-        uint64_t* w = T.snapw + so;
-        for (int c0 = w0; c0 < w1; c0 += WORDS) {
-            const int c1 = c0 + WORDS < w1 ? c0 + WORDS : w1;
-            for (int k = threadIdx.x; k < c1 - c0; k += NT) sw[k] = 0ull;
-            __syncthreads();
-            const int tb = 64 * c0, te = 64 * c1 < npt ? 64 * c1 : npt;
-            const int per = (te - tb + NT - 1) / NT;
-            int t = tb + (int)threadIdx.x * per;
-            const int t1 = t + per < te ? t + per : te;
-            if (t < t1) {
-                int a, bb;
-                tp_pair_of(t, a, bb);
-                for (; t < t1; ++t) {
-                    if (tp_snap_hit(seg, c9, h, a, bb)) atomicOr(&sw[(t >> 6) - c0], 1ull << (t & 63));
-                    if (++bb == a) { ++a; bb = 0; }
-                }
-            }
-            __syncthreads();
-            for (int k = threadIdx.x; k < c1 - c0; k += NT) w[c0 + k] = sw[k];
-            __syncthreads();
-        }
-#ifdef ZDX_WALK_PROFILE
-        if (threadIdx.x == 0 && it < 8192 && b == 0) {
-            g_topo_pairs[4 * it] = S;
-            g_topo_pairs[4 * it + 1] = (long long)(wall_clock64() - pa_t0);
-        }
-#endif
     }
 }
 
@@ -2428,36 +2284,41 @@ void launch_topo_zero(const DPairs& P, const TopoBufs& T, uint8_t* cur_active, i
     hipLaunchKernelGGL(k_topo_zero, dim3(g), dim3(256), 0, s, P, T, cur_active, stamp);
 }
 
+// Pass A of the pairs with few segments (P.topo_small)
+static void launch_pass_a_small(const DPairs& P, const DMeshes& M, const DBodies& B, const TopoBufs& T, hipStream_t s) {
+    hipLaunchKernelGGL((k_tp_pass_a<PA_SMALL_THREADS, PA_SMALL_WORDS, 1>), dim3((unsigned)T.pass_groups * 4),
+                       dim3(PA_SMALL_THREADS),
+                       (size_t)pass_a_lds_bytes(PA_SMALL_THREADS, PA_SMALL_WORDS, TOPO_BIG_SEGS), s, P, M, B, T,
+                       (int32_t)TOPO_BIG_SEGS);
+}
+// ... and of the others with their extra units (MODE 2), or of all (MODE 0)
+template <int MODE>
+static void launch_pass_a_big(const DPairs& P, const DMeshes& M, const DBodies& B, const TopoBufs& T, hipStream_t s) {
+    hipLaunchKernelGGL((k_tp_pass_a<PA_THREADS, PA_WORDS, MODE>), dim3((unsigned)T.pass_groups), dim3(PA_THREADS),
+                       (size_t)pass_a_lds_bytes(PA_THREADS, PA_WORDS, PA_SEGS), s, P, M, B, T, (int32_t)PA_SEGS);
+}
 static void launch_pass_a(const DPairs& P, const DMeshes& M, const DBodies& B, const TopoBufs& T, hipStream_t s,
                           bool zeroed = false, hipStream_t side = nullptr, hipEvent_t ev_fork = nullptr,
                           hipEvent_t ev_join = nullptr) {
     if (!zeroed) launch_fill_u64(T.top, 0ull, 5, s);
     hipLaunchKernelGGL(k_tp_alloc, dim3((unsigned)((T.pass_groups + 255) / 256 * 4)), dim3(256), 0, s, P, T);
     if (P.topo_big) {
-        // the pairs with few segments in small workgroups (many per CU) and
-        // the big ones with their extra units in 1024-thread workgroups; with
-        // a side stream the two launches run side by side
+        // the pairs with few segments in small workgroups, the big ones with their
+        // extra units in larger workgroups; with a side stream the two
+        // launches run side by side
         const bool fork = side && ev_fork && ev_join;
         hipStream_t sb = fork ? side : s;
         if (fork) {
             (void)hipEventRecord(ev_fork, s);
             (void)hipStreamWaitEvent(side, ev_fork, 0);
         }
-        hipLaunchKernelGGL((k_tp_pass_a<TP_PASS_A_THREADS, TP_PASS_A_KEYS, TP_PASS_A_WORDS, 2>),
-                           dim3((unsigned)T.pass_groups), dim3(TP_PASS_A_THREADS),
-                           84 * TP_PASS_A_SEGS + TP_PASS_A_KEYS + 8 * TP_PASS_A_WORDS, sb, P, M, B, T,
-                           (int32_t)TP_PASS_A_SEGS);
+        launch_pass_a_big<2>(P, M, B, T, sb);
         hipLaunchKernelGGL(k_tp_snap_cc, dim3(256), dim3(CC_THREADS), 0, sb, P, T);
         if (fork) (void)hipEventRecord(ev_join, side);
-        constexpr int SK = TOPO_BIG_SEGS * TOPO_BIG_SEGS, SW = 64;
-        hipLaunchKernelGGL((k_tp_pass_a<256, SK, SW, 1>), dim3((unsigned)T.pass_groups * 4), dim3(256),
-                           84 * TOPO_BIG_SEGS + SK + 8 * SW, s, P, M, B, T, (int32_t)TOPO_BIG_SEGS);
+        launch_pass_a_small(P, M, B, T, s);
         if (fork) (void)hipStreamWaitEvent(s, ev_join, 0);
     } else {
-        hipLaunchKernelGGL((k_tp_pass_a<TP_PASS_A_THREADS, TP_PASS_A_KEYS, TP_PASS_A_WORDS, 0>),
-                           dim3((unsigned)T.pass_groups), dim3(TP_PASS_A_THREADS),
-                           84 * TP_PASS_A_SEGS + TP_PASS_A_KEYS + 8 * TP_PASS_A_WORDS, s, P, M, B, T,
-                           (int32_t)TP_PASS_A_SEGS);
+        launch_pass_a_big<0>(P, M, B, T, s);
     }
 }
 
@@ -2483,10 +2344,7 @@ void launch_topo_sim(const DPairs& P, const DMeshes& M, const DBodies& B, const 
     hipLaunchKernelGGL(k_tp_alloc, dim3((unsigned)((T.pass_groups + 255) / 256 * 4)), dim3(256), 0, s, P, T);
     (void)hipEventRecord(ev_fork, s);
     (void)hipStreamWaitEvent(side, ev_fork, 0);
-    hipLaunchKernelGGL((k_tp_pass_a<TP_PASS_A_THREADS, TP_PASS_A_KEYS, TP_PASS_A_WORDS, 2>),
-                       dim3((unsigned)T.pass_groups), dim3(TP_PASS_A_THREADS),
-                       84 * TP_PASS_A_SEGS + TP_PASS_A_KEYS + 8 * TP_PASS_A_WORDS, side, P, M, B, T,
-                       (int32_t)TP_PASS_A_SEGS);
+    launch_pass_a_big<2>(P, M, B, T, side);
     hipLaunchKernelGGL(k_tp_snap_cc, dim3(256), dim3(CC_THREADS), 0, side, P, T);
     (void)hipEventRecord(ev_cc, side);
     const int64_t gs = T.nthreads - WALK_BIG_GROUPS;
@@ -2496,9 +2354,7 @@ void launch_topo_sim(const DPairs& P, const DMeshes& M, const DBodies& B, const 
     hipLaunchKernelGGL(k_tp_walk_bcd_sim<1>, dim3((unsigned)WALK_BIG_GROUPS), dim3(64), T.lds_bytes, side, P, M, B,
                        mat, H, Tb, sp, T.lds_bytes, 2);
     (void)hipEventRecord(ev_join, side);
-    constexpr int SK = TOPO_BIG_SEGS * TOPO_BIG_SEGS, SW = 64;
-    hipLaunchKernelGGL((k_tp_pass_a<256, SK, SW, 1>), dim3((unsigned)T.pass_groups * 4), dim3(256),
-                       84 * TOPO_BIG_SEGS + SK + 8 * SW, s, P, M, B, T, (int32_t)TOPO_BIG_SEGS);
+    launch_pass_a_small(P, M, B, T, s);
     // the small pairs' walks with the LDS their largest pair needs, so that
     // many more of them fit a CU at once
     const int Ss = TOPO_BIG_SEGS - 1;
