@@ -133,7 +133,7 @@ zdx_status zdx_contact_pairs_noalloc(zdx_ctx* ctx, const zdx_pair_in* pairs, int
                                      const zdx_contact_opts* opts, zdx_pair_out* out);
 
 /* Device time of the last zdx_contact_pairs call on this context (no
- * reference counterpart), from HIP events on the context's stream: out[0]
+ * reference counterpart), from the device clock at the stages' starts: out[0]
  * transform of the bodies, out[1] narrow phase (work ordering, cull, sweep,
  * exact tests, compaction) of the attempt that fitted the buffers, out[2]
  * topology and loop records, all in ms; out[3] narrow-phase attempts (1 when

@@ -194,9 +194,11 @@ struct zdx_ctx {
     // third stream: pass A of the many-segment pairs beside that of the others
     hipStream_t stream3 = nullptr;
     hipEvent_t ev_fork3 = nullptr, ev_join3 = nullptr, ev_cc3 = nullptr;
-    // timing events of the per-pair call: transform, narrow phase (the
-    // attempt that fitted), topology -- start and end of each
-    hipEvent_t ev_api[6] = {};
+    // the per-pair call's pinned host memory (API_PIN_BYTES: its input, a
+    // header, the output slots) and the device's address of it
+    char *pin = nullptr, *pin_dev = nullptr;
+    double clock_khz = 100000.0;   // the device clock that the calls' stamps count
+    // transform, narrow phase (the attempt that fitted), topology
     double api_ms[3] = {0.0, 0.0, 0.0};
     int32_t api_attempts = 0;
     std::string err;
@@ -227,10 +229,12 @@ struct zdx_ctx {
         DBuf<NarrowItem> items;
         DBuf<PairItem> pitems;
         DBuf<double> seg_tmp;
+        DBuf<unsigned long long> stamps;
         DBuf<int64_t> seg_off, tri_checks, tri_tests;
         DBuf<int32_t> nseg, tri_hits, tri_scanned;
         DBuf<double> arena;
         DBuf<int32_t> list_i;
+
         DBuf<float> list_f;
         DBuf<int32_t> hits, hit_tri, hit_flag;
         DBuf<unsigned long long> hit_top;
@@ -254,7 +258,7 @@ struct zdx_ctx {
         template <class F>
         void each_buf(F&& f) {
             f(pairs_in); f(mesh); f(state); f(wv_off); f(wt_off); f(wv); f(aabb); f(nondeg); f(pi); f(pj); f(order);
-            f(npairs); f(status); f(items); f(pitems); f(seg_tmp); f(seg_off); f(tri_checks); f(tri_tests); f(nseg); f(tri_hits);
+            f(npairs); f(status); f(items); f(pitems); f(seg_tmp); f(stamps); f(seg_off); f(tri_checks); f(tri_tests); f(nseg); f(tri_hits);
             f(tri_scanned); f(arena); f(list_i); f(list_f); f(hits); f(hit_tri); f(hit_flag); f(hit_top); f(hit_off);
             f(queue); f(heavy); f(bcnt); f(bcur); f(ncontrib); f(comps); f(loops_raw); f(tstatus); f(topo_list); f(topo_n);
             f(status2); f(rec); f(vtx); f(prov); f(ej); f(vj); f(ljac); f(pk_loop_off); f(pk_seg_off);
@@ -272,7 +276,7 @@ struct zdx_ctx {
     } api, api_na;
     // wall-contact queries (zdx_wall_contacts)
     struct WallQ {
-        DBuf<int32_t> mesh, nondeg, isrc, status;
+        DBuf<int32_t> mesh, nondeg, isrc;
         DBuf<double> state, wv, aabb, tris, normals, scr, out;
         DBuf<int64_t> wv_off, wt_off;
     } wq;
@@ -410,6 +414,19 @@ zdx_status guard(zdx_ctx* ctx, F&& f) {
         if (ctx) ctx->err = e.what();
         return ZDX_INTERNAL;
     }
+}
+// A call that ends by an error leaves nothing running that still reads its
+// pinned input.
+template <class F>
+zdx_status guard_drained(zdx_ctx* c, F&& f) {
+    return guard(c, [&] {
+        try {
+            f();
+        } catch (...) {
+            (void)hipStreamSynchronize(c->stream);
+            throw;
+        }
+    });
 }
 
 // Device memory of zdx_contact_pairs_noalloc: one array per GPU, made by the
@@ -1161,25 +1178,48 @@ void contact_pairs_impl(zdx_ctx* c, zdx_ctx::Api& A, const zdx_pair_in* pairs, i
             out->n_loops_total = out->n_vtx_total = out->n_seg_total = 0;
             return;
         }
-        // the pair records go to the device as they are; bodies, poses and
-        // world-vertex offsets are expanded there
-        A.pairs_in.ensure((size_t)n);
-        HIPC(hipMemcpyAsync(A.pairs_in.p, pairs, (size_t)n * sizeof(zdx_pair_in), hipMemcpyHostToDevice, st));
+        // the pair records go to the device as they are, with the bodies' first
+        // world vertices and triangles, through the context's pinned memory
+        // when they fit there; bodies and poses are expanded there
+        ApiBegin K0{};
+        K0.n = n;
+        std::vector<int64_t> off_v, off_t;
+        const bool pinned = (int64_t)n * (int64_t)sizeof(zdx_pair_in) + 2 * 8 * ((int64_t)nb + 1) <= API_PIN_IN;
+        int64_t *wvo = (int64_t*)c->pin, *wto = wvo + nb + 1;
+        if (!pinned) {
+            off_v.resize((size_t)nb + 1); off_t.resize((size_t)nb + 1);
+            wvo = off_v.data(); wto = off_t.data();
+        }
+        int64_t at = 0;
+        av = 0;
+        for (int b = 0; b < nb; ++b) {
+            const HostMesh& m = c->meshes[b & 1 ? pairs[b >> 1].mesh_b : pairs[b >> 1].mesh_a].h;
+            wvo[b] = av; wto[b] = at;
+            av += (int64_t)(m.verts.size() / 3);
+            at += (int64_t)(m.tri_idx.size() / 3);
+        }
+        wvo[nb] = av; wto[nb] = at;
         A.mesh.ensure(nb); A.state.ensure(16 * (size_t)nb); A.wv_off.ensure((size_t)nb + 1); A.wt_off.ensure((size_t)nb + 1);
+        if (pinned) {
+            const size_t o = 2 * 8 * ((size_t)nb + 1);
+            std::memcpy(c->pin + o, pairs, (size_t)n * sizeof(zdx_pair_in));
+            K0.wvo_in = (const int64_t*)c->pin_dev; K0.wto_in = K0.wvo_in + nb + 1;
+            K0.in = (const zdx_pair_in*)(c->pin_dev + o);
+        } else {
+            A.pairs_in.upload(pairs, (size_t)n, st);
+            A.wv_off.upload(wvo, (size_t)nb + 1, st);
+            A.wt_off.upload(wto, (size_t)nb + 1, st);
+            K0.in = A.pairs_in.p;
+        }
+        K0.mesh = A.mesh.p; K0.state = A.state.p; K0.wvo = A.wv_off.p; K0.wto = A.wt_off.p;
         DMeshes M = c->dmeshes();
-        launch_api_bodies(A.pairs_in.p, n, M, A.mesh.p, A.state.p, A.wv_off.p, A.wt_off.p, st);
         A.wv.ensure(3 * (size_t)av); A.aabb.ensure(6 * (size_t)nb); A.nondeg.ensure(nb);
         DBodies B;
         B.n = nb; B.mesh = A.mesh.p; B.state = A.state.p; B.wv_off = A.wv_off.p; B.wt_off = A.wt_off.p;
         B.wv = A.wv.p; B.nondeg = A.nondeg.p; B.aabb = A.aabb.p;
-        HIPC(hipEventRecord(c->ev_api[0], st));
-        launch_transform(B, M, st);
-        HIPC(hipEventRecord(c->ev_api[1], st));
         A.pi.ensure(n); A.pj.ensure(n); A.npairs.ensure(1); A.status.ensure(1); A.order.ensure(n); A.items.ensure(n);
-        A.pitems.ensure(n);
+        A.pitems.ensure(n); A.stamps.ensure(4);
         A.status2.ensure(1);
-        launch_iota_pairs(A.pi.p, A.pj.p, n, st);
-        launch_fill_i32(A.npairs.p, n, 1, st);
         A.seg_off.ensure(n); A.tri_checks.ensure(n); A.tri_tests.ensure(n); A.nseg.ensure(n); A.tri_hits.ensure(n); A.tri_scanned.ensure(n);
         A.queue.ensure(NARROW_COUNTERS); A.heavy.ensure(n); A.bcnt.ensure(64); A.bcur.ensure(64);
         A.hit_off.ensure(n); A.hit_top.ensure(HIT_SHARDS * HIT_TOP_STRIDE);
@@ -1193,6 +1233,9 @@ void contact_pairs_impl(zdx_ctx* c, zdx_ctx::Api& A, const zdx_pair_in* pairs, i
             A.list_f.ensure((size_t)groups * 12 * c->max_tris);
         }
         const bool want_vtx = out->loop_vtx != nullptr;
+        ApiHead* const head = (ApiHead*)(c->pin + API_PIN_IN);
+        auto slot = [&](char* base, int k) { return base + API_PIN_IN + 4096 + k * API_SLOT; };
+        auto transform_ms = [&] { c->api_ms[0] = (double)(int64_t)(head->clock[1] - head->clock[0]) / c->clock_khz; };
         for (int attempt = 0; attempt < 10; ++attempt) {
             c->api_attempts = attempt + 1;
             A.arena.ensure((size_t)A.hit_cap * 6);
@@ -1200,9 +1243,14 @@ void contact_pairs_impl(zdx_ctx* c, zdx_ctx::Api& A, const zdx_pair_in* pairs, i
             A.hit_flag.ensure((size_t)A.hit_cap);
             if (c->clusters) A.seg_tmp.ensure(6 * (size_t)A.hit_cap);
             const bool sens = opts->sensitivities != 0;
+            NarrowCfg nc{API_GROUP, 4, groups, batched ? 1 : 0, std::min(persistent_groups(c, 4), (n + 3) / 4)};
+            nc.side = c->stream3; nc.ev_fork = c->ev_fork3; nc.ev_join = c->ev_join3;
+            nc.few = n <= PAIRS_FEW;
+            // the order matters where pairs wait for each other
+            const bool ordered = batched && !(nc.few && c->clusters);
             DPairs P{};
-            P.cap = n; P.n = A.npairs.p; P.pi = A.pi.p; P.pj = A.pj.p; P.order = batched ? A.order.p : nullptr;
-            P.items = batched ? A.items.p : nullptr;
+            P.cap = n; P.n = A.npairs.p; P.pi = A.pi.p; P.pj = A.pj.p; P.order = ordered ? A.order.p : nullptr;
+            P.items = ordered ? A.items.p : nullptr;
             P.pitems = A.pitems.p; P.seg_tmp = A.seg_tmp.p;
             P.seg_off = A.seg_off.p; P.nseg = A.nseg.p; P.tri_checks = A.tri_checks.p; P.tri_tests = A.tri_tests.p;
             P.tri_hits = A.tri_hits.p; P.tri_scanned = A.tri_scanned.p; P.arena = A.arena.p; P.arena_cap = A.hit_cap;
@@ -1218,22 +1266,33 @@ void contact_pairs_impl(zdx_ctx* c, zdx_ctx::Api& A, const zdx_pair_in* pairs, i
                 A.prov.ensure((size_t)A.hit_cap * 4);
                 P.prov = A.prov.p;
             }
-            launch_fill_i32(A.status.p, 0, 1, st);
-            launch_fill_i32(A.topo_n.p, 0, 1, st);
-            HIPC(hipEventRecord(c->ev_api[2], st));
-            if (batched) launch_lpt_order(P, M, B, A.order.p, A.bcnt.p, A.bcur.p, n, st);
-            NarrowCfg nc{API_GROUP, 4, groups, batched ? 1 : 0, std::min(persistent_groups(c, 4), (n + 3) / 4)};
-            nc.side = c->stream3; nc.ev_fork = c->ev_fork3; nc.ev_join = c->ev_join3;
-            nc.few = n <= PAIRS_FEW;
-            launch_narrow(B, M, P, nc, A.list_i.p, A.list_f.p, A.stage_cap, c->max_tris, A.queue.p, st);
-            HIPC(hipEventRecord(c->ev_api[3], st));
-            int32_t status = 0;
-            HIPC(hipMemcpyAsync(&status, A.status.p, 4, hipMemcpyDeviceToHost, st));
-            HIPC(hipStreamSynchronize(st));
-            if (status & (ST_STAGE | ST_HITS)) {
+            A.tw.ensure_bump();
+            int32_t* const z[ApiBegin::NZ] = {A.status.p, A.topo_n.p, (int32_t*)A.queue.p, A.bcnt.p, A.bcur.p,
+                                              (int32_t*)A.hit_top.p, (int32_t*)A.tw.top.p};
+            const int64_t zn[ApiBegin::NZ] = {1, 1, NARROW_COUNTERS, 64, 64, 2 * HIT_SHARDS * HIT_TOP_STRIDE, 10};
+            for (int k = 0; k < ApiBegin::NZ; ++k) { K0.zero[k] = z[k]; K0.n0[k] = zn[k]; }
+            K0.pi = A.pi.p; K0.pj = A.pj.p; K0.npairs = A.npairs.p;
+            K0.ncontrib = A.ncontrib.p; K0.comps = A.comps.p; K0.raw = A.loops_raw.p; K0.tstatus = A.tstatus.p;
+            launch_api_begin(K0, st);
+            if (K0.in) launch_transform(B, M, st, nullptr, nullptr, 0, A.stamps.p);
+            K0.in = nullptr;
+            if (ordered) launch_lpt_order(P, M, B, A.order.p, A.bcnt.p, A.bcur.p, n, st, true, A.stamps.p + 1);
+            launch_narrow(B, M, P, nc, A.list_i.p, A.list_f.p, A.stage_cap, c->max_tris, A.queue.p, st, true,
+                          ordered ? nullptr : A.stamps.p + 1);
+            auto narrow_grew = [&](int32_t status) {
                 if (status & ST_STAGE) A.stage_cap *= 4;
                 if (status & ST_HITS) A.hit_cap = grown_hit_cap(A.hit_top.p, P.hit_shards, A.hit_cap);
-                continue;
+                return (status & (ST_STAGE | ST_HITS)) != 0;
+            };
+            // before the topology's buffers grow, whether the narrow phase's
+            // were large enough for them to be sized
+            if (!lim.may_allocate || A.tw.cell9.n < 9 * (size_t)A.hit_cap ||
+                (sens && A.vj.n < 72 * (size_t)A.hit_cap)) {
+                HIPC(hipMemcpyAsync(&head->status, A.status.p, 4, hipMemcpyDeviceToHost, st));
+                HIPC(hipMemcpyAsync(head->clock, A.stamps.p, 16, hipMemcpyDeviceToHost, st));
+                HIPC(hipStreamSynchronize(st));
+                if (attempt == 0) transform_ms();
+                if (narrow_grew(head->status)) continue;
             }
             // topology with the minimal-energy force
             TopoBufs T{};
@@ -1259,17 +1318,52 @@ void contact_pairs_impl(zdx_ctx* c, zdx_ctx::Api& A, const zdx_pair_in* pairs, i
                 T.ej = A.ej.p; T.vj = A.vj.p; T.ljac = A.ljac.p;
             }
             T.rec = A.rec.p; T.vtx = want_vtx ? A.vtx.p : nullptr;
-            HIPC(hipEventRecord(c->ev_api[4], st));
-            launch_topo_zero(P, T, nullptr, n, st);
+            T.stamp_alloc = A.stamps.p + 2;
             launch_topo_api(P, M, B, T, opts->split_contacts, st);
-            HIPC(hipEventRecord(c->ev_api[5], st));
-            HIPC(hipMemcpyAsync(&status, A.status.p, 4, hipMemcpyDeviceToHost, st));
-            HIPC(hipStreamSynchronize(st));
-            for (int k = 0; k < 3; ++k) {
-                float ms = 0.0f;
-                HIPC(hipEventElapsedTime(&ms, c->ev_api[2 * k], c->ev_api[2 * k + 1]));
-                c->api_ms[k] = ms;
+            // pack on the device: small outputs straight to their slots in host
+            // memory, the others to device memory, one copy each
+            const bool want_jac = sens && out->loop_jac;
+            const bool want_seg = out->segments != nullptr;
+            const bool columns = 8 * ((int64_t)n + 1) <= API_SLOT;
+            ApiPack K{};
+            K.n = n; K.lmax = T.lmax; K.vmax = T.vmax;
+            K.status = A.status.p; K.stamps = A.stamps.p;
+            K.head = (ApiHead*)(c->pin_dev + API_PIN_IN);
+            K.nloops = A.ncontrib.p; K.nseg = A.nseg.p; K.seg_off = A.seg_off.p;
+            K.comps = A.comps.p; K.raw = A.loops_raw.p; K.tri_checks = A.tri_checks.p;
+            K.rec = A.rec.p; K.ljac = want_jac ? A.ljac.p : nullptr; K.vtx = want_vtx ? A.vtx.p : nullptr;
+            K.arena = A.arena.p;
+            A.pk_loop_off.ensure((size_t)n + 1); A.pk_seg_off.ensure((size_t)n + 1);
+            A.pk_pvtx.ensure((size_t)n + 1); A.pk_tot.ensure(3);
+            K.loop_off = A.pk_loop_off.p; K.seg_out_off = A.pk_seg_off.p; K.pvtx_off = A.pk_pvtx.p;
+            K.totals = A.pk_tot.p;
+            K.loop_cap = std::max<int64_t>(0, std::min<int64_t>(out->loop_cap, (int64_t)n * T.lmax));
+            K.vtx_cap = want_vtx ? std::max<int64_t>(0, std::min<int64_t>(out->vtx_cap, (int64_t)n * T.vmax)) : 0;
+            K.seg_cap = want_seg ? std::max<int64_t>(0, std::min<int64_t>(out->seg_cap, A.hit_cap)) : 0;
+            K.want_seg = want_seg;
+            auto output = [&](auto& o, auto& buf, int k, int64_t words, bool want) {
+                using W = std::remove_reference_t<decltype(*o.host)>;
+                if (!want) return;
+                o.host = (W*)slot(c->pin_dev, k);
+                if (words * (int64_t)sizeof(W) > API_SLOT) o.dev = buf.ensure((size_t)words);
+            };
+            output(K.rec_out, A.pk_rec, 6, K.loop_cap * 28, out->loop_rec != nullptr);
+            output(K.ljac_out, A.pk_ljac, 7, K.loop_cap * 72, want_jac);
+            output(K.vtx_out, A.pk_vtx, 8, K.vtx_cap * 3, want_vtx);
+            output(K.vtx_off_out, A.pk_vtx_off, 9, K.loop_cap + 1, want_vtx);
+            output(K.seg_out, A.pk_seg, 10, K.seg_cap * 6, want_seg);
+            if (columns) {
+                K.h_loop_off = (int32_t*)slot(c->pin_dev, 0); K.h_seg_off = (int32_t*)slot(c->pin_dev, 1);
+                K.h_nseg = (int32_t*)slot(c->pin_dev, 2); K.h_comps = (int32_t*)slot(c->pin_dev, 3);
+                K.h_raw = (int32_t*)slot(c->pin_dev, 4); K.h_checks = (int64_t*)slot(c->pin_dev, 5);
             }
+            launch_api_pack(K, st);
+            HIPC(hipStreamSynchronize(st));
+            const int32_t status = head->status;
+            if (attempt == 0) transform_ms();
+            for (int k = 1; k < 3; ++k)
+                c->api_ms[k] = (double)(int64_t)(head->clock[k + 1] - head->clock[k]) / c->clock_khz;
+            if (narrow_grew(status)) continue;
             if (status & ST_TOPO) {
                 int32_t ts = 0;
                 launch_or_i32(A.tstatus.p, n, A.status2.p, st);
@@ -1282,32 +1376,7 @@ void contact_pairs_impl(zdx_ctx* c, zdx_ctx::Api& A, const zdx_pair_in* pairs, i
                 if (!lo && !vo && !grown) throw ApiError{ZDX_CAPACITY, "contact topology exceeded its edge capacity"};
                 continue;
             }
-            // pack on the device, then one copy per output array
-            const bool want_jac = sens && out->loop_jac;
-            const bool want_seg = out->segments != nullptr;
-            ApiPack K{};
-            K.n = n; K.lmax = T.lmax; K.vmax = T.vmax;
-            K.nloops = A.ncontrib.p; K.nseg = A.nseg.p; K.seg_off = A.seg_off.p;
-            K.rec = A.rec.p; K.ljac = want_jac ? A.ljac.p : nullptr; K.vtx = want_vtx ? A.vtx.p : nullptr;
-            K.arena = A.arena.p;
-            A.pk_loop_off.ensure((size_t)n + 1); A.pk_seg_off.ensure((size_t)n + 1);
-            A.pk_pvtx.ensure((size_t)n + 1); A.pk_tot.ensure(3);
-            K.loop_off = A.pk_loop_off.p; K.seg_out_off = A.pk_seg_off.p; K.pvtx_off = A.pk_pvtx.p;
-            K.totals = A.pk_tot.p;
-            K.loop_cap = std::max<int64_t>(0, std::min<int64_t>(out->loop_cap, (int64_t)n * T.lmax));
-            K.vtx_cap = want_vtx ? std::max<int64_t>(0, std::min<int64_t>(out->vtx_cap, (int64_t)n * T.vmax)) : 0;
-            K.seg_cap = want_seg ? std::max<int64_t>(0, std::min<int64_t>(out->seg_cap, A.hit_cap)) : 0;
-            if (out->loop_rec) { A.pk_rec.ensure((size_t)K.loop_cap * 28 + 1); K.rec_out = A.pk_rec.p; }
-            if (want_jac) { A.pk_ljac.ensure((size_t)K.loop_cap * 72 + 1); K.ljac_out = A.pk_ljac.p; }
-            if (want_vtx) {
-                A.pk_vtx.ensure((size_t)K.vtx_cap * 3 + 1); K.vtx_out = A.pk_vtx.p;
-                A.pk_vtx_off.ensure((size_t)K.loop_cap + 1); K.vtx_off_out = A.pk_vtx_off.p;
-            }
-            if (want_seg) { A.pk_seg.ensure((size_t)K.seg_cap * 6 + 1); K.seg_out = A.pk_seg.p; }
-            launch_api_pack(K, st);
-            int64_t tot[3] = {0, 0, 0};
-            HIPC(hipMemcpyAsync(tot, A.pk_tot.p, sizeof(tot), hipMemcpyDeviceToHost, st));
-            HIPC(hipStreamSynchronize(st));
+            const int64_t* tot = head->totals;
             out->n_loops_total = tot[0];
             out->n_vtx_total = tot[1];
             out->n_seg_total = tot[2];
@@ -1315,25 +1384,36 @@ void contact_pairs_impl(zdx_ctx* c, zdx_ctx::Api& A, const zdx_pair_in* pairs, i
                 throw ApiError{ZDX_CAPACITY, "zdx_pair_out capacity too small (see n_*_total)"};
             if (tot[0] >= ((int64_t)1 << 31) || tot[1] >= ((int64_t)1 << 31) || tot[2] >= ((int64_t)1 << 31))
                 throw ApiError{ZDX_CAPACITY, "more than 2^31 loops, loop vertices or segments in one call"};
-            auto d2h = [&](void* dst, const void* src, size_t bytes) {
-                if (bytes) HIPC(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st));
+            bool copies = false;
+            auto fetch = [&](void* dst, int k, bool here, const void* src, int64_t bytes) {
+                if (!dst || bytes <= 0) return;
+                if (here) {
+                    std::memcpy(dst, slot(c->pin, k), (size_t)bytes);
+                } else {
+                    HIPC(hipMemcpyAsync(dst, src, (size_t)bytes, hipMemcpyDeviceToHost, st));
+                    copies = true;
+                }
             };
-            d2h(out->loop_offset, A.pk_loop_off.p, 4 * ((size_t)n + 1));
-            if (out->tri_checks) d2h(out->tri_checks, A.tri_checks.p, 8 * (size_t)n);
-            if (out->n_segments) d2h(out->n_segments, A.nseg.p, 4 * (size_t)n);
-            if (out->n_comps) d2h(out->n_comps, A.comps.p, 4 * (size_t)n);
-            if (out->n_loops_raw) d2h(out->n_loops_raw, A.loops_raw.p, 4 * (size_t)n);
-            if (out->loop_rec) d2h(out->loop_rec, A.pk_rec.p, 8 * 28 * (size_t)tot[0]);
-            if (want_jac) d2h(out->loop_jac, A.pk_ljac.p, 8 * 72 * (size_t)tot[0]);
+            auto rows = [&](void* dst, int k, const void* src, int64_t bytes) {
+                fetch(dst, k, bytes <= API_SLOT, src, bytes);
+            };
+            // the large ones are under way while the host copies the others
+            if (out->loop_rec) rows(out->loop_rec, 6, A.pk_rec.p, 8 * 28 * tot[0]);
+            if (want_jac) rows(out->loop_jac, 7, A.pk_ljac.p, 8 * 72 * tot[0]);
             if (want_vtx) {
-                d2h(out->vtx_offset, A.pk_vtx_off.p, 4 * ((size_t)tot[0] + 1));
-                d2h(out->loop_vtx, A.pk_vtx.p, 8 * 3 * (size_t)tot[1]);
+                rows(out->vtx_offset, 9, A.pk_vtx_off.p, 4 * (tot[0] + 1));
+                rows(out->loop_vtx, 8, A.pk_vtx.p, 8 * 3 * tot[1]);
             }
             if (want_seg) {
-                d2h(out->seg_offset, A.pk_seg_off.p, 4 * ((size_t)n + 1));
-                d2h(out->segments, A.pk_seg.p, 8 * 6 * (size_t)tot[2]);
+                fetch(out->seg_offset, 1, columns, A.pk_seg_off.p, 4 * ((int64_t)n + 1));
+                rows(out->segments, 10, A.pk_seg.p, 8 * 6 * tot[2]);
             }
-            HIPC(hipStreamSynchronize(st));
+            fetch(out->loop_offset, 0, columns, A.pk_loop_off.p, 4 * ((int64_t)n + 1));
+            fetch(out->tri_checks, 5, columns, A.tri_checks.p, 8 * (int64_t)n);
+            fetch(out->n_segments, 2, columns, A.nseg.p, 4 * (int64_t)n);
+            fetch(out->n_comps, 3, columns, A.comps.p, 4 * (int64_t)n);
+            fetch(out->n_loops_raw, 4, columns, A.loops_raw.p, 4 * (int64_t)n);
+            if (copies) HIPC(hipStreamSynchronize(st));
             return;
         }
         throw ApiError{ZDX_CAPACITY, "per-pair buffers did not fit after repeated growth"};
@@ -1366,7 +1446,13 @@ zdx_status zdx_create(zdx_ctx** out, int32_t device) {
         HIPC(hipEventCreateWithFlags(&c->ev_fork3, hipEventDisableTiming));
         HIPC(hipEventCreateWithFlags(&c->ev_join3, hipEventDisableTiming));
         HIPC(hipEventCreateWithFlags(&c->ev_cc3, hipEventDisableTiming));
-        for (auto& e : c->ev_api) HIPC(hipEventCreate(&e));
+        HIPC(hipHostMalloc((void**)&c->pin, (size_t)API_PIN_BYTES, hipHostMallocCoherent));
+        void* pd = nullptr;
+        HIPC(hipHostGetDevicePointer(&pd, c->pin, 0));
+        c->pin_dev = (char*)pd;
+        int khz = 0;
+        if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device) == hipSuccess && khz > 0)
+            c->clock_khz = (double)khz;
         // this device's copy of the no-allocation scratch
         void* sp = nullptr;
         HIPC(hipGetSymbolAddress(&sp, HIP_SYMBOL(scratch)));
@@ -1380,6 +1466,7 @@ zdx_status zdx_create(zdx_ctx** out, int32_t device) {
         }
     });
     if (st != ZDX_OK) {
+        if (c->pin) (void)hipHostFree(c->pin);
         delete c;
         return st;
     }
@@ -1393,8 +1480,7 @@ void zdx_destroy(zdx_ctx* c) {
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     if (c->stream2) (void)hipStreamSynchronize(c->stream2);
     if (c->stream3) (void)hipStreamSynchronize(c->stream3);
-    for (auto& e : c->ev_api)
-        if (e) (void)hipEventDestroy(e);
+    if (c->pin) (void)hipHostFree(c->pin);
     if (c->ev_fork3) (void)hipEventDestroy(c->ev_fork3);
     if (c->ev_join3) (void)hipEventDestroy(c->ev_join3);
     if (c->ev_cc3) (void)hipEventDestroy(c->ev_cc3);
@@ -1439,13 +1525,13 @@ zdx_status zdx_mesh_register(zdx_ctx* c, const double* tris, int32_t T, int32_t 
 zdx_status zdx_contact_pairs(zdx_ctx* c, const zdx_pair_in* pairs, int32_t n, const zdx_contact_opts* opts,
                              zdx_pair_out* out) {
     if (!c || (!pairs && n > 0) || n < 0 || !opts || !out || !out->loop_offset) return ZDX_BAD_ARG;
-    return guard(c, [&] { contact_pairs_impl(c, c->api, pairs, n, opts, out, CallLimits{}); });
+    return guard_drained(c, [&] { contact_pairs_impl(c, c->api, pairs, n, opts, out, CallLimits{}); });
 }
 
 zdx_status zdx_contact_pairs_noalloc(zdx_ctx* c, const zdx_pair_in* pairs, int32_t n, const zdx_contact_opts* opts,
                                      zdx_pair_out* out) {
     if (!c || (!pairs && n > 0) || n < 0 || !opts || !out || !out->loop_offset) return ZDX_BAD_ARG;
-    return guard(c, [&] {
+    return guard_drained(c, [&] {
         if (!c->scratch_dev) throw ApiError{ZDX_INTERNAL, "no-allocation scratch address not set up"};
         // every call starts from the front of this device's scratch array
         c->na_arena.reset();
@@ -1462,7 +1548,7 @@ zdx_status zdx_wall_contacts(zdx_ctx* c, const zdx_body_pose* bodies, int32_t n,
                              const double* wall_normals, int32_t n_tris, int32_t jac, double* out) {
     if (!c || n < 0 || n_tris < 0 || ((n > 0 && n_tris > 0) && (!bodies || !wall_tris || !wall_normals || !out)))
         return ZDX_BAD_ARG;
-    return guard(c, [&] {
+    return guard_drained(c, [&] {
         HIPC(hipSetDevice(c->device));
         if (n == 0 || n_tris == 0) return;
         for (int b = 0; b < n; ++b)
@@ -1471,15 +1557,29 @@ zdx_status zdx_wall_contacts(zdx_ctx* c, const zdx_body_pose* bodies, int32_t n,
         c->sync_meshes();
         hipStream_t st = c->stream;
         auto& Q = c->wq;
-        std::vector<int32_t> mesh(n);
-        std::vector<double> state(16 * (size_t)n, 0.0);
-        std::vector<int64_t> wvo(n + 1), wto(n + 1);
+        // the call's input, one part after the other, in the context's pinned
+        // memory when it fits there (one launch moves it), else copied
+        const int64_t nq = (int64_t)n * n_tris;
+        const int64_t out_words = 32 * nq + 1;   // the last one: the status
+        const size_t part[6] = {128 * (size_t)n, 8 * ((size_t)n + 1), 8 * ((size_t)n + 1), 72 * (size_t)n_tris,
+                                24 * (size_t)n_tris, 4 * (size_t)n};
+        size_t at_part[7] = {0};
+        for (int k = 0; k < 6; ++k) at_part[k + 1] = at_part[k] + part[k];
+        const bool pinned = (int64_t)at_part[6] <= API_PIN_IN && 8 * out_words <= API_SLOTS * API_SLOT;
+        std::vector<char> host;
+        if (!pinned) host.resize(at_part[6]);
+        char* in = pinned ? c->pin : host.data();
+        double* state = (double*)in;
+        int64_t *wvo = (int64_t*)(in + at_part[1]), *wto = (int64_t*)(in + at_part[2]);
+        int32_t* mesh = (int32_t*)(in + at_part[5]);
+        std::memcpy(in + at_part[3], wall_tris, part[3]);
+        std::memcpy(in + at_part[4], wall_normals, part[4]);
         int64_t av = 0, at = 0;
         int32_t tmax = 1;
         for (int b = 0; b < n; ++b) {
             mesh[b] = bodies[b].mesh;
-            for (int k = 0; k < 3; ++k) state[16 * (size_t)b + k] = bodies[b].pos[k];
-            for (int k = 0; k < 4; ++k) state[16 * (size_t)b + 3 + k] = bodies[b].quat[k];
+            for (int k = 0; k < 16; ++k)
+                state[16 * (size_t)b + k] = k < 3 ? bodies[b].pos[k] : (k < 7 ? bodies[b].quat[k - 3] : 0.0);
             wvo[b] = av; wto[b] = at;
             av += (int64_t)(c->meshes[mesh[b]].h.verts.size() / 3);
             const int32_t T = (int32_t)(c->meshes[mesh[b]].h.tri_idx.size() / 3);
@@ -1487,13 +1587,23 @@ zdx_status zdx_wall_contacts(zdx_ctx* c, const zdx_body_pose* bodies, int32_t n,
             tmax = std::max(tmax, T);
         }
         wvo[n] = av; wto[n] = at;
-        Q.mesh.upload(mesh.data(), n, st);
-        Q.state.upload(state.data(), state.size(), st);
-        Q.wv_off.upload(wvo.data(), n + 1, st);
-        Q.wt_off.upload(wto.data(), n + 1, st);
+        Q.state.ensure(16 * (size_t)n); Q.wv_off.ensure((size_t)n + 1); Q.wt_off.ensure((size_t)n + 1);
+        Q.tris.ensure(9 * (size_t)n_tris); Q.normals.ensure(3 * (size_t)n_tris); Q.mesh.ensure(n);
+        Q.out.ensure((size_t)out_words);
+        int32_t* const status_dev = (int32_t*)(Q.out.p + 32 * nq);
+        void* const dst[6] = {Q.state.p, Q.wv_off.p, Q.wt_off.p, Q.tris.p, Q.normals.p, Q.mesh.p};
+        CopyParts K{};
+        for (int k = 0; k < 6; ++k) {
+            if (!pinned) HIPC(hipMemcpyAsync(dst[k], in + at_part[k], part[k], hipMemcpyHostToDevice, st));
+            else {
+                K.src[k] = (const int32_t*)(c->pin_dev + at_part[k]);
+                K.dst[k] = (int32_t*)dst[k];
+                K.n[k] = (int64_t)(part[k] / 4);
+            }
+        }
+        K.zero = status_dev;
+        launch_copy_parts(K, st);
         Q.wv.ensure(3 * (size_t)av); Q.aabb.ensure(6 * (size_t)n); Q.nondeg.ensure(n);
-        Q.tris.upload(wall_tris, 9 * (size_t)n_tris, st);
-        Q.normals.upload(wall_normals, 3 * (size_t)n_tris, st);
         DBodies B;
         B.n = n; B.mesh = Q.mesh.p; B.state = Q.state.p; B.wv_off = Q.wv_off.p; B.wt_off = Q.wt_off.p;
         B.wv = Q.wv.p; B.nondeg = Q.nondeg.p; B.aabb = Q.aabb.p;
@@ -1501,18 +1611,24 @@ zdx_status zdx_wall_contacts(zdx_ctx* c, const zdx_body_pose* bodies, int32_t n,
         launch_transform(B, M, st);
         // section points: at most one per edge slot of the body mesh
         const int32_t cap = 3 * tmax;
-        const int64_t nq = (int64_t)n * n_tris;
         Q.scr.ensure((size_t)nq * (size_t)(3 * (int64_t)cap + 32 * (int64_t)(cap + 8)));
         Q.isrc.ensure((size_t)nq * (size_t)(cap + 1));
-        Q.out.ensure(32 * (size_t)nq);
-        Q.status.ensure(1);
-        launch_fill_i32(Q.status.p, 0, 1, st);
         launch_wall_query(B, M, n, Q.tris.p, Q.normals.p, n_tris, jac ? 1 : 0, cap, Q.scr.p, Q.isrc.p, Q.out.p,
-                          Q.status.p, st);
+                          status_dev, st);
         int32_t status = 0;
-        HIPC(hipMemcpyAsync(&status, Q.status.p, 4, hipMemcpyDeviceToHost, st));
-        HIPC(hipMemcpyAsync(out, Q.out.p, 32 * 8 * (size_t)nq, hipMemcpyDeviceToHost, st));
-        HIPC(hipStreamSynchronize(st));
+        if (pinned) {
+            char* const o = c->pin + API_PIN_IN + 4096;
+            CopyParts R{};
+            R.src[0] = (const int32_t*)Q.out.p; R.dst[0] = (int32_t*)(c->pin_dev + API_PIN_IN + 4096); R.n[0] = 2 * out_words;
+            launch_copy_parts(R, st);
+            HIPC(hipStreamSynchronize(st));
+            std::memcpy(&status, o + 256 * nq, 4);
+            std::memcpy(out, o, 256 * (size_t)nq);
+        } else {
+            HIPC(hipMemcpyAsync(&status, status_dev, 4, hipMemcpyDeviceToHost, st));
+            HIPC(hipMemcpyAsync(out, Q.out.p, 256 * (size_t)nq, hipMemcpyDeviceToHost, st));
+            HIPC(hipStreamSynchronize(st));
+        }
         if (status & 2) throw ApiError{ZDX_INTERNAL, "wall contact derivative disagreed with the contact"};
         if (status) throw ApiError{ZDX_INTERNAL, "wall section exceeded its point capacity"};
     });

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "../../include/zdx.h"
 #include "zdx_internal.h"
 
 namespace zdx {
@@ -258,42 +259,87 @@ void launch_fold_integrate(int32_t n, const double* state_in, double* state_out,
 // leaves; nullptr skips them)
 void launch_fill_i32(int32_t* p, int32_t v, int64_t n, hipStream_t s);
 void launch_fill_u64(unsigned long long* p, unsigned long long v, int64_t n, hipStream_t s);
-void launch_iota_pairs(int32_t* pi, int32_t* pj, int32_t n, hipStream_t s);
 
 // Output of the per-pair call packed on the device, so that each array
 // reaches the caller in one copy: per-pair loop, vertex and segment offsets
 // (exclusive scans), then the accepted loops' records (28 doubles), their
 // Jacobians (72, optional), their vertices (optional) and the segments
 // (optional) back to back in pair order.  Optional outputs are NULL.
+// The per-pair call's host memory (pinned, one block per context): the
+// caller's pairs go to the device from its input part, small outputs come back
+// through its slots, written by the device, so that a call waits for the
+// device once.
+constexpr int64_t API_PIN_IN = (int64_t)1 << 20;
+constexpr int64_t API_SLOT = (int64_t)512 << 10;   // an output array up to this size; a larger one is copied
+constexpr int API_SLOTS = 11;
+constexpr int API_PACK_ONE = 64;                   // calls up to this many pairs are packed by the scanning workgroup
+struct ApiHead {
+    int32_t status, pad;
+    int64_t totals[3];               // loops, vertices, segments
+    unsigned long long clock[4];     // start of the transform, of the narrow phase, of the topology, its end
+};
+constexpr int64_t API_PIN_BYTES = API_PIN_IN + 4096 + API_SLOTS * API_SLOT;
+static_assert(sizeof(ApiHead) <= 4096, "the header's place");
+template <class T>
+struct ApiOut {
+    T *host = nullptr, *dev = nullptr;
+};
 struct ApiPack {
     int32_t n;                 // pairs
     int32_t lmax, vmax;        // per-pair slots of rec / ljac and of vtx
+    const int32_t* status;     // nothing is packed unless 0
+    const unsigned long long* stamps;   // the first three of head->clock
+    ApiHead* head;             // host memory
     const int32_t* nloops;     // accepted loops per pair
     const int32_t* nseg;       // segments per pair
+    const int32_t *comps, *raw;
+    const int64_t* tri_checks;
     const int64_t* seg_off;    // the pair's first segment in the arena
     const double* rec;         // n * lmax * 28
     const double* ljac;        // n * lmax * 72
-    const double* vtx;         // n * vmax * 3
+    const double* vtx;         // n * vmax * 3, or nullptr: not wanted
     const double* arena;       // segments, 6 doubles each
     int32_t* loop_off;         // n + 1
     int32_t* seg_out_off;      // n + 1
     int64_t* pvtx_off;         // n + 1: first vertex of each pair's loops
     int64_t* totals;           // loops, vertices, segments
-    double* rec_out;           // loop_cap * 28
-    double* ljac_out;          // loop_cap * 72
-    double* vtx_out;           // vtx_cap * 3
-    int32_t* vtx_off_out;      // loop_cap + 1
-    double* seg_out;           // seg_cap * 6
+    ApiOut<double> rec_out;    // loop_cap * 28
+    ApiOut<double> ljac_out;   // loop_cap * 72
+    ApiOut<double> vtx_out;    // vtx_cap * 3
+    ApiOut<int32_t> vtx_off_out;   // loop_cap + 1
+    ApiOut<double> seg_out;    // seg_cap * 6
+    bool want_seg;
     int64_t loop_cap, vtx_cap, seg_cap;   // rows of the *_out arrays: nothing is written past them
+    // the per-pair columns' slots (all or none: h_loop_off nullptr)
+    int32_t *h_loop_off, *h_seg_off, *h_nseg, *h_comps, *h_raw;
+    int64_t* h_checks;
 };
 void launch_api_pack(const ApiPack& k, hipStream_t s);
-// Bodies of the per-pair call from the caller's pair records (zdx_pair_in,
-// copied to the device as they are, `in`): body 2p is pair p's A, 2p + 1 its
-// B.  Writes mesh ids, state rows (pos, quat, the rest 0) and each body's
-// first world vertex and triangle (exclusive scans over the meshes' counts,
-// 2n + 1 entries: the last holds the totals).
-void launch_api_bodies(const void* in, int32_t n, const DMeshes& M, int32_t* mesh, double* state, int64_t* wv_off,
-                       int64_t* wt_off, hipStream_t s);
+// Moves up to six arrays of words between device memory and a call's pinned
+// memory, and clears one word.
+struct CopyParts {
+    const int32_t* src[6];
+    int32_t* dst[6];
+    int64_t n[6];
+    int32_t* zero;             // optional
+};
+void launch_copy_parts(const CopyParts& k, hipStream_t s);
+// Start of an attempt of the per-pair call.  Body 2p is pair p's A, 2p + 1 its
+// B: mesh ids, state rows (pos, quat, the rest 0) and, when given, each body's
+// first world vertex and triangle.
+struct ApiBegin {
+    static constexpr int NZ = 7;
+    int32_t n;
+    int32_t* zero[NZ];         // cleared words
+    int64_t n0[NZ];
+    int32_t *pi, *pj, *npairs, *ncontrib, *comps, *raw, *tstatus;
+    const zdx_pair_in* in;     // nullptr: bodies already there
+    const int64_t *wvo_in, *wto_in;
+    int32_t* mesh;
+    double* state;
+    int64_t *wvo, *wto;
+};
+void launch_api_begin(const ApiBegin& k, hipStream_t s);
 // Wall contacts of bodies against wall triangles (the per-triangle part of
 // the reference's particle-wall contact, src/main.cpp:2325-2369, without its
 // bounding-sphere and box pre-tests): one wave per (body b, triangle t);

@@ -994,7 +994,8 @@ __device__ inline void make_item(const DPairs& P, const DMeshes& M, const DBodie
     P.items[slot] = it;
 }
 // the items in pair order (no work ordering)
-__global__ void __launch_bounds__(256) k_pair_items(DPairs P, DMeshes M, DBodies B) {
+__global__ void __launch_bounds__(256) k_pair_items(DPairs P, DMeshes M, DBodies B, unsigned long long* stamp) {
+    stamp_here(stamp);
     const int n = *P.n;
     for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x) make_item(P, M, B, p, p);
 }
@@ -1878,143 +1879,163 @@ __global__ void __launch_bounds__(256) k_fold_integrate(int32_t n, const double*
     store_body(sout + 16 * (int64_t)i, b);
 }
 
-__global__ void k_iota_pairs(int32_t* pi, int32_t* pj, int32_t n) {
-    int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p < n) { pi[p] = 2 * p; pj[p] = 2 * p + 1; }
+// The per-pair call's packed output, one pair per wave: each array goes to the
+// caller-visible host memory when it fits its slot there, else to device
+// memory (ApiOut).  A pair whose rows would pass an output's capacity writes
+// nothing to that output (the host then reports the totals and the call fails
+// with ZDX_CAPACITY).
+template <class T>
+__device__ inline T* api_dst(const ApiOut<T>& o, int64_t rows, int per) {
+    return o.host && rows * per * (int64_t)sizeof(T) <= API_SLOT ? o.host : o.dev;
 }
-
-
-// Offsets of the per-pair call's packed output: one workgroup scans the
-// pairs 1024 at a time (loops, loop vertices, segments of each pair) with a
-// carry between chunks.
+__device__ inline void api_pack_pair(const ApiPack& k, int64_t p, int lane) {
+    const int64_t L = k.totals[0];
+    const int nl = k.nloops[p];
+    const int64_t lo = k.loop_off[p];
+    double* rec = api_dst(k.rec_out, L, 28);
+    double* ljac = api_dst(k.ljac_out, L, 72);
+    if (lo + nl <= k.loop_cap) {
+        if (rec)
+            for (int64_t e = lane; e < 28 * (int64_t)nl; e += WAVE) rec[28 * lo + e] = k.rec[(p * k.lmax) * 28 + e];
+        if (ljac)
+            for (int64_t e = lane; e < 72 * (int64_t)nl; e += WAVE) ljac[72 * lo + e] = k.ljac[(p * k.lmax) * 72 + e];
+    }
+    if (k.vtx) {
+        double* vtx = api_dst(k.vtx_out, k.totals[1], 3);
+        int32_t* off = api_dst(k.vtx_off_out, L + 1, 1);
+        const int64_t vo = k.pvtx_off[p];
+        const int64_t nv = k.pvtx_off[p + 1] - vo;
+        if (lane == 0 && lo + nl <= k.loop_cap) {
+            int64_t acc = vo;
+            for (int l = 0; l < nl; ++l) {
+                off[lo + l] = (int32_t)acc;
+                acc += (int64_t)k.rec[(p * k.lmax + l) * 28 + 24];
+            }
+            if (p == k.n - 1) off[lo + nl] = (int32_t)acc;
+        }
+        if (vo + nv <= k.vtx_cap)
+            for (int64_t e = lane; e < 3 * nv; e += WAVE) vtx[3 * vo + e] = k.vtx[(p * k.vmax) * 3 + e];
+    }
+    if (k.want_seg) {
+        double* seg = api_dst(k.seg_out, k.totals[2], 6);
+        const int64_t so = k.seg_out_off[p];
+        const int ns = k.nseg[p];
+        if (so + ns <= k.seg_cap)
+            for (int64_t e = lane; e < 6 * (int64_t)ns; e += WAVE) seg[6 * so + e] = k.arena[6 * k.seg_off[p] + e];
+    }
+    // the per-pair columns
+    if (k.h_loop_off) {
+        if (lane < (p == k.n - 1 ? 2 : 1)) {
+            k.h_loop_off[p + lane] = k.loop_off[p + lane];
+            k.h_seg_off[p + lane] = k.seg_out_off[p + lane];
+        }
+        if (lane == 0) {
+            k.h_checks[p] = k.tri_checks[p];
+            k.h_nseg[p] = k.nseg[p];
+            k.h_comps[p] = k.comps[p];
+            k.h_raw[p] = k.raw[p];
+        }
+    }
+}
+// Its offsets: one workgroup scans the pairs 1024 at a time (loops, loop
+// vertices, segments of each pair) with a carry between chunks, writes the
+// call's header, and packs the pairs of a small call itself.  Nothing is
+// packed when the call's status is not zero (it is run again).
 __global__ void __launch_bounds__(1024) k_api_scan(ApiPack k) {
-    __shared__ long long sh[3][1024];
-    __shared__ long long carry[3];
-    const int t = threadIdx.x;
-    if (t < 3) carry[t] = 0;
-    __syncthreads();
-    for (int base = 0; base < k.n; base += 1024) {
+    constexpr int NW = 1024 / WAVE;
+    __shared__ long long s_w[3][NW];
+    const int t = threadIdx.x, lane = lane_id(), wid = t / WAVE;
+    const int status = *k.status;
+    const unsigned long long now = wall_clock64();
+    long long carry[3] = {0, 0, 0};
+    for (int base = 0; base < k.n && status == 0; base += 1024) {
         const int p = base + t;
-        long long v[3] = {0, 0, 0};
+        long long v[3] = {0, 0, 0}, x[3];
         if (p < k.n) {
             v[0] = k.nloops[p];
-            for (int l = 0; l < k.nloops[p]; ++l) v[1] += (long long)k.rec[((int64_t)p * k.lmax + l) * 28 + 24];
+            for (int l = 0; l < (int)v[0]; ++l) v[1] += (long long)k.rec[((int64_t)p * k.lmax + l) * 28 + 24];
             v[2] = k.nseg[p];
         }
-        for (int c = 0; c < 3; ++c) sh[c][t] = v[c];
+        for (int c = 0; c < 3; ++c) {
+            x[c] = v[c];
+            for (int d = 1; d < WAVE; d <<= 1) {
+                const long long y = __shfl_up(x[c], d, WAVE);
+                if (lane >= d) x[c] += y;
+            }
+            if (lane == WAVE - 1) s_w[c][wid] = x[c];
+        }
         __syncthreads();
-        for (int off = 1; off < 1024; off <<= 1) {
-            long long a[3];
-            for (int c = 0; c < 3; ++c) a[c] = t >= off ? sh[c][t - off] : 0;
-            __syncthreads();
-            for (int c = 0; c < 3; ++c) sh[c][t] += a[c];
-            __syncthreads();
+        for (int c = 0; c < 3; ++c) {
+            long long before = carry[c];
+            for (int q = 0; q < NW; ++q) {
+                before += q < wid ? s_w[c][q] : 0;
+                carry[c] += s_w[c][q];
+            }
+            x[c] += before;
         }
         if (p < k.n) {
-            k.loop_off[p] = (int32_t)(carry[0] + sh[0][t] - v[0]);
-            k.pvtx_off[p] = carry[1] + sh[1][t] - v[1];
-            k.seg_out_off[p] = (int32_t)(carry[2] + sh[2][t] - v[2]);
+            k.loop_off[p] = (int32_t)(x[0] - v[0]);
+            k.pvtx_off[p] = x[1] - v[1];
+            k.seg_out_off[p] = (int32_t)(x[2] - v[2]);
         }
-        __syncthreads();
-        if (t < 3) carry[t] += sh[t][1023];
         __syncthreads();
     }
     if (t == 0) {
         k.loop_off[k.n] = (int32_t)carry[0];
         k.pvtx_off[k.n] = carry[1];
         k.seg_out_off[k.n] = (int32_t)carry[2];
-        k.totals[0] = carry[0];
-        k.totals[1] = carry[1];
-        k.totals[2] = carry[2];
-        if (k.vtx_off_out && carry[0] <= k.loop_cap) k.vtx_off_out[carry[0]] = (int32_t)carry[1];
+        for (int c = 0; c < 3; ++c) k.totals[c] = k.head->totals[c] = carry[c];
+        k.head->status = status;
+        for (int c = 0; c < 3; ++c) k.head->clock[c] = k.stamps[c];
+        k.head->clock[3] = now;
     }
-}
-
-// One wave per pair moves its rows to the packed positions; a pair whose
-// rows would pass an output's capacity writes nothing to that output (the
-// host then reports the totals and the call fails with ZDX_CAPACITY).
-__global__ void __launch_bounds__(256) k_api_pack(ApiPack k) {
-    const int lane = threadIdx.x & 63;
-    const int64_t nw = (int64_t)gridDim.x * (blockDim.x >> 6);
-    for (int64_t p = blockIdx.x * (int64_t)(blockDim.x >> 6) + (threadIdx.x >> 6); p < k.n; p += nw) {
-        const int nl = k.nloops[p];
-        const int64_t lo = k.loop_off[p];
-        if (lo + nl <= k.loop_cap) {
-            if (k.rec_out)
-                for (int64_t e = lane; e < 28 * (int64_t)nl; e += 64)
-                    k.rec_out[28 * lo + e] = k.rec[(p * k.lmax) * 28 + e];
-            if (k.ljac_out)
-                for (int64_t e = lane; e < 72 * (int64_t)nl; e += 64)
-                    k.ljac_out[72 * lo + e] = k.ljac[(p * k.lmax) * 72 + e];
-        }
-        if (k.vtx_out) {
-            const int64_t vo = k.pvtx_off[p];
-            const int64_t nv = k.pvtx_off[p + 1] - vo;
-            if (lane == 0 && lo + nl <= k.loop_cap) {
-                int64_t acc = vo;
-                for (int l = 0; l < nl; ++l) {
-                    k.vtx_off_out[lo + l] = (int32_t)acc;
-                    acc += (int64_t)k.rec[(p * k.lmax + l) * 28 + 24];
-                }
-            }
-            if (vo + nv <= k.vtx_cap)
-                for (int64_t e = lane; e < 3 * nv; e += 64) k.vtx_out[3 * vo + e] = k.vtx[(p * k.vmax) * 3 + e];
-        }
-        if (k.seg_out) {
-            const int64_t so = k.seg_out_off[p];
-            const int ns = k.nseg[p];
-            if (so + ns <= k.seg_cap)
-                for (int64_t e = lane; e < 6 * (int64_t)ns; e += 64) k.seg_out[6 * so + e] = k.arena[6 * k.seg_off[p] + e];
-        }
-    }
-}
-
-__global__ void __launch_bounds__(1024) k_api_bodies(const zdx_pair_in* in, int32_t n, DMeshes M, int32_t* mesh,
-                                                    double* state, int64_t* wvo, int64_t* wto) {
-    __shared__ long long sh[2][1024];
-    __shared__ long long carry[2];
-    const int t = threadIdx.x;
-    const int64_t nb = 2 * (int64_t)n;
-    if (t < 2) carry[t] = 0;
+    if (k.n > API_PACK_ONE || status != 0) return;
     __syncthreads();
-    for (int64_t base = 0; base < nb; base += 1024) {
-        const int64_t b = base + t;
-        long long v[2] = {0, 0};
-        if (b < nb) {
-            const zdx_pair_in& q = in[b >> 1];
-            const int side = (int)(b & 1);
-            const int m = side ? q.mesh_b : q.mesh_a;
-            const double* pos = side ? q.pos_b : q.pos_a;
-            const double* qu = side ? q.quat_b : q.quat_a;
-            mesh[b] = m;
-            double* st = state + 16 * b;
-            st[0] = pos[0]; st[1] = pos[1]; st[2] = pos[2];
-            st[3] = qu[0]; st[4] = qu[1]; st[5] = qu[2]; st[6] = qu[3];
-            for (int k = 7; k < 16; ++k) st[k] = 0.0;
-            v[0] = M.nverts[m];
-            v[1] = M.ntris[m];
-        }
-        for (int c = 0; c < 2; ++c) sh[c][t] = v[c];
-        __syncthreads();
-        for (int off = 1; off < 1024; off <<= 1) {
-            long long a[2];
-            for (int c = 0; c < 2; ++c) a[c] = t >= off ? sh[c][t - off] : 0;
-            __syncthreads();
-            for (int c = 0; c < 2; ++c) sh[c][t] += a[c];
-            __syncthreads();
-        }
-        if (b < nb) {
-            wvo[b] = carry[0] + sh[0][t] - v[0];
-            wto[b] = carry[1] + sh[1][t] - v[1];
-        }
-        __syncthreads();
-        if (t < 2) carry[t] += sh[t][1023];
-        __syncthreads();
+    for (int p = wid; p < k.n; p += NW) api_pack_pair(k, p, lane);
+}
+__global__ void __launch_bounds__(256) k_api_pack(ApiPack k) {
+    if (*k.status != 0) return;
+    const int64_t nw = (int64_t)gridDim.x * (blockDim.x / WAVE);
+    for (int64_t p = blockIdx.x * (int64_t)(blockDim.x / WAVE) + threadIdx.x / WAVE; p < k.n; p += nw)
+        api_pack_pair(k, p, lane_id());
+}
+
+// The start of an attempt of the per-pair call: the counters and per-pair
+// outputs that its kernels expect cleared and, on the first, the bodies of the
+// caller's pairs (read in place when they lie in the call's host memory).
+__global__ void __launch_bounds__(256) k_api_begin(ApiBegin k) {
+    const int64_t at = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
+    for (int z = 0; z < ApiBegin::NZ; ++z)
+        for (int64_t e = at; e < k.n0[z]; e += step) k.zero[z][e] = 0;
+    for (int64_t p = at; p < k.n; p += step) {
+        k.ncontrib[p] = k.comps[p] = k.raw[p] = k.tstatus[p] = 0;
+        k.pi[p] = 2 * (int32_t)p;
+        k.pj[p] = 2 * (int32_t)p + 1;
     }
-    if (t == 0) {
-        wvo[nb] = carry[0];
-        wto[nb] = carry[1];
+    if (at == 0) *k.npairs = k.n;
+    if (!k.in) return;
+    // a word of a state row per thread: a wave reads whole records
+    const int64_t nb = 2 * (int64_t)k.n;
+    for (int64_t e = at; e < 16 * nb; e += step) {
+        const int64_t b = e >> 4;
+        const int c = (int)(e & 15);
+        const zdx_pair_in& q = k.in[b >> 1];
+        const bool side = (b & 1) != 0;
+        double v = 0.0;
+        if (c < 3) v = side ? q.pos_b[c] : q.pos_a[c];
+        else if (c < 7) v = side ? q.quat_b[c - 3] : q.quat_a[c - 3];
+        k.state[e] = v;
+        if (c == 7) k.mesh[b] = side ? q.mesh_b : q.mesh_a;
+        if (c == 8 && k.wvo_in) k.wvo[b] = k.wvo_in[b];
+        if (c == 9 && k.wto_in) k.wto[b] = k.wto_in[b];
     }
+}
+
+__global__ void __launch_bounds__(256) k_copy_parts(CopyParts k) {
+    const int64_t at = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
+    for (int p = 0; p < 6; ++p)
+        for (int64_t e = at; e < k.n[p]; e += step) k.dst[p][e] = k.src[p][e];
+    if (at == 0 && k.zero) *k.zero = 0;
 }
 
 __global__ void __launch_bounds__(64) k_wall_query(DBodies B, DMeshes M, int32_t n_bodies, const double* tris,
@@ -2162,8 +2183,11 @@ static void launch_pairs(const DBodies& B, const DMeshes& M, const DPairs& P, co
                          unsigned int* q, hipStream_t s, int wave_groups, int32_t wave_tests,
                          unsigned long long* stamp) {
     // without the work ordering (plain mode) the items in pair order
-    if (!P.order)
-        hipLaunchKernelGGL(k_pair_items, dim3(std::max(1, std::min(nblk(P.cap, 256), 1024))), dim3(256), 0, s, P, M, B);
+    if (!P.order) {
+        hipLaunchKernelGGL(k_pair_items, dim3(std::max(1, std::min(nblk(P.cap, 256), 1024))), dim3(256), 0, s, P, M, B,
+                           stamp);
+        stamp = nullptr;
+    }
     auto group = [&](auto kernel, int bs, int back, hipStream_t gs) {
         const int32_t* count = back < 0 ? P.n : (const int32_t*)(q + (back ? NQ_HEAVY_BACK : NQ_HEAVY));
         hipLaunchKernelGGL(kernel, dim3(cfg.groups), dim3(bs), (size_t)pairs_group_lds_bytes(bs), gs, B, M, P,
@@ -2368,8 +2392,8 @@ void launch_topo_sim(const DPairs& P, const DMeshes& M, const DBodies& B, const 
 }
 void launch_topo_api(const DPairs& P, const DMeshes& M, const DBodies& B, const TopoBufs& T, int32_t split,
                      hipStream_t s) {
+    launch_pass_a(P, M, B, T, s, true);
     if (T.ej) hipLaunchKernelGGL(k_tp_endpoint_jac, dim3((unsigned)T.pass_groups), dim3(256), 0, s, P, M, B, T);
-    launch_pass_a(P, M, B, T, s);
     hipLaunchKernelGGL(k_tp_walk_b, dim3((unsigned)T.nthreads), dim3(64), T.lds_bytes, s, P, M, B, T, split,
                        T.lds_bytes);
     hipLaunchKernelGGL(k_tp_pass_c, dim3((unsigned)T.pass_groups), dim3(256), 0, s, P, M, B, T);
@@ -2409,27 +2433,26 @@ void launch_fill_u64(unsigned long long* p, unsigned long long v, int64_t n, hip
     if (g > 4096) g = 4096;
     hipLaunchKernelGGL(k_fill_u64, dim3(g), dim3(256), 0, s, p, v, n);
 }
-void launch_iota_pairs(int32_t* pi, int32_t* pj, int32_t n, hipStream_t s) {
-    if (n <= 0) return;
-    hipLaunchKernelGGL(k_iota_pairs, dim3(nblk(n, 256)), dim3(256), 0, s, pi, pj, n);
-}
-
 void launch_api_pack(const ApiPack& k, hipStream_t s) {
     if (k.n <= 0) return;
     hipLaunchKernelGGL(k_api_scan, dim3(1), dim3(1024), 0, s, k);
-    hipLaunchKernelGGL(k_api_pack, dim3(std::min(nblk(k.n, 4), 4096)), dim3(256), 0, s, k);
+    if (k.n > API_PACK_ONE) hipLaunchKernelGGL(k_api_pack, dim3(std::min(nblk(k.n, 4), 4096)), dim3(256), 0, s, k);
 }
 
-void launch_api_bodies(const void* in, int32_t n, const DMeshes& M, int32_t* mesh, double* state, int64_t* wv_off,
-                       int64_t* wt_off, hipStream_t s) {
-    if (n <= 0) return;
-    hipLaunchKernelGGL(k_api_bodies, dim3(1), dim3(1024), 0, s, (const zdx_pair_in*)in, n, M, mesh, state, wv_off,
-                       wt_off);
+void launch_api_begin(const ApiBegin& k, hipStream_t s) {
+    const int64_t most = std::max<int64_t>(k.in ? 32 * (int64_t)k.n : k.n, 4096);
+    hipLaunchKernelGGL(k_api_begin, dim3(std::min(nblk(most, 256), 1024)), dim3(256), 0, s, k);
 }
 
 void launch_or_i32(const int32_t* v, int32_t n, int32_t* out, hipStream_t s) {
     hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, s, out, 0, nullptr, (int64_t)1);
     if (n > 0) hipLaunchKernelGGL(k_or_i32, dim3(std::min(nblk(n, 256), 1024)), dim3(256), 0, s, v, n, out);
+}
+
+void launch_copy_parts(const CopyParts& k, hipStream_t s) {
+    int64_t most = 1;
+    for (int64_t n : k.n) most = std::max(most, n);
+    hipLaunchKernelGGL(k_copy_parts, dim3(std::min(nblk(most, 256), 1024)), dim3(256), 0, s, k);
 }
 
 void launch_wall_query(const DBodies& B, const DMeshes& M, int32_t n_bodies, const double* tris, const double* normals,
