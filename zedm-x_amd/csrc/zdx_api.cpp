@@ -951,11 +951,6 @@ void enqueue_step(zdx_sim* s, int par, bool batched) {
     DPairs P = s->dpairs(par, batched);
     TopoBufs T = s->topobufs();
     HistBufs H = s->hist(par);
-    // batched: the work ordering's scatter pass zeroes the topology's per-pair
-    // outputs, and k_tp_alloc stamps the narrow phase's end
-    if (batched)
-        launch_lpt_order(P, M, B, s->d_order.p, s->d_bcnt.p, s->d_bcur.p, s->pair_cap, st, true, kt + 2, &T,
-                         H.cur_active);
     NarrowCfg nc = s->ncfg;
     nc.use_queue = batched ? 1 : 0;
     nc.groups = g_narrow;
@@ -971,6 +966,16 @@ void enqueue_step(zdx_sim* s, int par, bool batched) {
         P.topo_big = P.topo_small = P.n_big = P.n_small = nullptr;
         T.lds_bytes = std::max(T.lds_bytes, TOPO_LDS_FEW);
     }
+    // the work items' pass zeroes the topology's per-pair outputs, and
+    // k_tp_alloc stamps the narrow phase's end
+    nc.items_made = s->ctx->clusters && (nc.few || !batched);
+    if (nc.items_made) {
+        P.order = nullptr;
+        launch_pair_items(P, M, B, T, H.cur_active, st, batched ? kt + 2 : nullptr);
+    } else if (batched) {
+        launch_lpt_order(P, M, B, s->d_order.p, s->d_bcnt.p, s->d_bcur.p, s->pair_cap, st, true, kt + 2, &T,
+                         H.cur_active);
+    }
     launch_narrow(B, M, P, nc, s->d_list_i.p, s->d_list_f.p, s->stage_cap, s->tmax, s->d_queue.p, st,
                   true, kt + 8);
     if (!batched) launch_stamp(kt + 3, st);   // batched: stamped by k_tp_alloc (no host read in between)
@@ -982,7 +987,7 @@ void enqueue_step(zdx_sim* s, int par, bool batched) {
         T.pass_groups = std::max<int64_t>(1, std::min<int64_t>(nt, T.pass_groups));
     }
     if (batched) T.stamp_alloc = kt + 3;
-    else launch_topo_zero(P, T, H.cur_active, s->pair_cap, st, nullptr);
+    else if (!nc.items_made) launch_topo_zero(P, T, H.cur_active, s->pair_cap, st, nullptr);
     launch_topo_sim(P, M, B, mat, H, T, s->sp, st, true, s->ctx->stream3, s->ctx->ev_fork3, s->ctx->ev_join3,
                     s->ctx->ev_cc3);
     if (walls) HIPC(hipStreamWaitEvent(st, s->ctx->ev_join, 0));

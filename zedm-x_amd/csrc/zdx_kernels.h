@@ -147,6 +147,7 @@ struct NarrowCfg {
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     // cluster path: few pairs (PAIRS_FEW), each by a workgroup at once
     bool few = false;
+    bool items_made = false;   // the work items are there (launch_pair_items), in pair order
 };
 // The most pairs that get a workgroup each at once: two workgroups of 512
 // threads fit on each of 256 CUs.
@@ -232,6 +233,11 @@ void launch_lpt_order(const DPairs& P, const DMeshes& M, const DBodies& B, int32
                       uint8_t* cur_active = nullptr);
 // zero outputs of every pair (the topology kernels then visit only the
 // pairs of P.topo_list); cur_active may be NULL
+// Work items in pair order and the topology's per-pair outputs cleared, for
+// few pairs on the cluster path: no pair waits for another, so the order
+// (launch_lpt_order) is left out.
+void launch_pair_items(const DPairs& P, const DMeshes& M, const DBodies& B, const TopoBufs& T, uint8_t* cur_active,
+                       hipStream_t s, unsigned long long* stamp = nullptr);
 void launch_topo_zero(const DPairs& P, const TopoBufs& T, uint8_t* cur_active, int32_t pair_cap, hipStream_t s,
                       unsigned long long* stamp = nullptr);
 // side/ev_fork/ev_join (optional, with P.topo_big): pass A of the many-segment

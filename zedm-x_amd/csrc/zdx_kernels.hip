@@ -698,6 +698,175 @@ __device__ inline bool near_any_wall(const WallBufs& W, const double* st, double
     return wall;
 }
 
+// The whole broad phase of at most BP_SMALL particles by one workgroup: every
+// pair takes the sphere test, one wave per particle's row; the rows are bit
+// masks, whose counts below a bit are the positions in the pair and adjacency
+// lists (partners in ascending order, as k_bp_fill sorts them).  Ten kernels
+// of 3 to 10 us and the gaps between them, 140 us for 64 bodies, are one of
+// 10 us; at 256 particles a wave still has only 64 tests of its 64 lanes.
+constexpr int BP_SMALL = 256;
+__global__ void __launch_bounds__(1024) k_bp_small(BroadPhaseBufs bp, NeedLists need, unsigned long long* kt0,
+                                                   StepZero z) {
+    constexpr int NW = 1024 / WAVE, KW = BP_SMALL / WAVE;
+    __shared__ double s_q[4][BP_SMALL];
+    __shared__ uint64_t s_m[BP_SMALL][KW];
+    __shared__ int s_all[BP_SMALL], s_low[BP_SMALL], s_po[BP_SMALL + 1], s_ao[BP_SMALL + 1], s_need[2];
+    const int tid = threadIdx.x, lane = lane_id(), wid = tid / WAVE, n = bp.n;
+    const uint64_t below = (1ull << lane) - 1ull;
+    if (kt0) {
+        if (tid == 0) *kt0 = (unsigned long long)wall_clock64();
+        for (int a = 0; a < 8; ++a)
+            if (z.i32[a])
+                for (int k = tid; k < z.n32[a]; k += 1024) z.i32[a][k] = 0;
+        for (int a = 0; a < 2; ++a)
+            if (z.u64[a])
+                for (int k = tid; k < z.n64[a]; k += 1024) z.u64[a][k] = 0ull;
+    }
+    if (tid < 2) s_need[tid] = 0;
+    if (tid < n) {
+        const double* p = bp.state + 16 * (int64_t)tid;
+        for (int k = 0; k < 3; ++k) s_q[k][tid] = p[k];
+        s_q[3][tid] = bp.radius[tid];
+    }
+    __threadfence();   // the cleared words come before what is stored or counted in them below
+    __syncthreads();
+    for (int i = wid; i < n; i += NW) {
+        const double xi = s_q[0][i], yi = s_q[1][i], zi = s_q[2][i], ri = s_q[3][i];
+        int all = 0, low = 0;
+#pragma unroll
+        for (int k = 0; k < KW; ++k) {
+            const int j = k * WAVE + lane;
+            bool on = false;
+            if (j < n && j != i) {
+                const double xj = s_q[0][j], yj = s_q[1][j], zj = s_q[2][j], rj = s_q[3][j];
+                const bool iflow = i < j;
+                const V3 pa = iflow ? v3(xi, yi, zi) : v3(xj, yj, zj);
+                const V3 pb = iflow ? v3(xj, yj, zj) : v3(xi, yi, zi);
+                const V3 dp = sub(pb, pa);
+                const double d2 = dot(dp, dp);
+                const double rs = iflow ? ri + rj : rj + ri;
+                on = !(d2 > rs * rs);
+            }
+            const uint64_t m = __ballot(on);
+            const int li = i - k * WAVE;   // bits below i of this word
+            if (lane == 0) s_m[i][k] = m;
+            all += __popcll(m);
+            low += __popcll(li <= 0 ? 0ull : (li >= WAVE ? m : m & ((1ull << li) - 1ull)));
+        }
+        if (lane == 0) { s_all[i] = all; s_low[i] = low; }
+    }
+    __syncthreads();
+    // exclusive prefixes of the upper and of all partners (first wave), the
+    // bounds' check, the need lists
+    if (wid == 0) {
+        int u[KW], a[KW], su = 0, sa = 0;
+#pragma unroll
+        for (int k = 0; k < KW; ++k) {
+            const int i = KW * lane + k;
+            a[k] = i < n ? s_all[i] : 0;
+            u[k] = i < n ? a[k] - s_low[i] : 0;
+            su += u[k];
+            sa += a[k];
+        }
+        int xu = su, xa = sa;
+        for (int d = 1; d < WAVE; d <<= 1) {
+            const int yu = __shfl_up(xu, d, WAVE), ya = __shfl_up(xa, d, WAVE);
+            if (lane >= d) { xu += yu; xa += ya; }
+        }
+        if (lane == WAVE - 1) { s_po[n] = xu; s_ao[n] = xa; }
+        xu -= su;
+        xa -= sa;
+#pragma unroll
+        for (int k = 0; k < KW; ++k) {
+            const int i = KW * lane + k;
+            if (i < n) {
+                s_po[i] = xu; s_ao[i] = xa;
+                bp.cnt_up[i] = u[k]; bp.cnt_all[i] = a[k];
+            }
+            xu += u[k];
+            xa += a[k];
+        }
+        // as bp_grid: finite bounds and largest radius
+        double v[7] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY, 0.0};
+        for (int i = lane; i < n; i += WAVE) {
+            for (int k = 0; k < 3; ++k) { v[k] = fmin(v[k], s_q[k][i]); v[3 + k] = fmax(v[3 + k], s_q[k][i]); }
+            v[6] = fmax(v[6], s_q[3][i]);
+        }
+        for (int d = 32; d >= 1; d >>= 1)
+            for (int k = 0; k < 7; ++k) {
+                const double o = __shfl_xor(v[k], d, WAVE);
+                v[k] = k < 3 ? fmin(v[k], o) : fmax(v[k], o);
+            }
+        const bool bad = !(isfinite(v[3] - v[0]) && isfinite(v[4] - v[1]) && isfinite(v[5] - v[2]) && isfinite(v[6]));
+        if (bad && lane == 0) atomicOr(bp.status, (int)ST_GRID);
+    }
+    if (need.list) {
+        bool nd = false, wall = false;
+        if (tid < n) {
+            wall = near_any_wall(need.W, bp.state + 16 * (int64_t)tid, bp.radius[tid]);
+            nd = wall || s_all[tid] > 0;
+        }
+        if (tid < BP_SMALL) {
+            const uint64_t bn = __ballot(nd), bw = __ballot(wall);
+            int on = 0, ow = 0;
+            if (lane == 0) {
+                on = atomicAdd(&s_need[0], __popcll(bn));
+                ow = atomicAdd(&s_need[1], __popcll(bw));
+            }
+            on = __shfl(on, 0, WAVE) + __popcll(bn & below);
+            ow = __shfl(ow, 0, WAVE) + __popcll(bw & below);
+            if (nd) need.list[on] = tid;
+            if (wall) need.wlist[ow] = tid;
+        }
+    }
+    __syncthreads();
+    const int np = s_po[n], na = s_ao[n];
+    const bool over = np > bp.pair_cap || na > bp.adj_cap;
+    if (tid == 0) {
+        if (over) atomicOr(bp.status, (int)ST_PAIRS);
+        *bp.n_pairs = over ? 0 : np;
+        *bp.n_adj = over ? 0 : na;
+        if (need.list) {
+            *need.n_list = s_need[0];
+            *need.n_wlist = s_need[1];
+        }
+    }
+    if (tid <= n) {
+        bp.pair_off[tid] = s_po[tid];
+        bp.adj_off[tid] = s_ao[tid];
+    }
+    if (over) return;
+    for (int i = wid; i < n; i += NW) {
+        const int po = s_po[i], ao = s_ao[i], low = s_low[i];
+        int before = 0;
+        for (int k = 0; k < KW; ++k) {
+            const uint64_t m = s_m[i][k];
+            if (m >> lane & 1ull) {
+                const int j = k * WAVE + lane, rank = before + __popcll(m & below);
+                int p;
+                if (j > i) {
+                    p = po + rank - low;
+                    bp.pi[p] = i;
+                    bp.pj[p] = j;
+                    bp.pkey[p] = ((int64_t)i << 32) | (int64_t)(uint32_t)j;
+                } else {
+                    // i's place among the upper partners of j
+                    int c = 0;
+                    for (int q = 0; q < KW; ++q) {
+                        const int li = i - q * WAVE;
+                        const uint64_t w = s_m[j][q];
+                        c += __popcll(li <= 0 ? 0ull : (li >= WAVE ? w : w & ((1ull << li) - 1ull)));
+                    }
+                    p = s_po[j] + c - s_low[j];
+                }
+                bp.adj_j[ao + rank] = j;
+                bp.adj_pair[ao + rank] = p;
+            }
+            before += __popcll(m);
+        }
+    }
+}
+
 // Particles in a candidate pair or near a wall triangle (list) and those near
 // a wall triangle (wlist), appended with one atomic per workgroup and list.
 // The order of the lists is free: the transform and the wall kernel write
@@ -994,10 +1163,22 @@ __device__ inline void make_item(const DPairs& P, const DMeshes& M, const DBodie
     P.items[slot] = it;
 }
 // the items in pair order (no work ordering)
-__global__ void __launch_bounds__(256) k_pair_items(DPairs P, DMeshes M, DBodies B, unsigned long long* stamp) {
+// (with tz, the topology's per-pair outputs start at zero too)
+__device__ inline void topo_zero_pair(const TopoBufs& T, uint8_t* cur_active, int p) {
+    T.ncontrib[p] = 0;
+    T.comps[p] = 0;
+    T.loops_raw[p] = 0;
+    T.tstatus[p] = 0;
+    if (cur_active) cur_active[p] = 0;
+}
+__global__ void __launch_bounds__(256) k_pair_items(DPairs P, DMeshes M, DBodies B, TopoBufs T, uint8_t* cur_active,
+                                                    int32_t tz, unsigned long long* stamp) {
     stamp_here(stamp);
     const int n = *P.n;
-    for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x) make_item(P, M, B, p, p);
+    for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x) {
+        if (tz) topo_zero_pair(T, cur_active, p);
+        make_item(P, M, B, p, p);
+    }
 }
 // order within a bucket is free (any order gives the same per-pair results)
 __global__ void __launch_bounds__(256) k_lpt_scatter(DPairs P, DMeshes M, DBodies B, const int32_t* bucket_cnt,
@@ -1031,14 +1212,7 @@ __global__ void __launch_bounds__(256) k_lpt_scatter(DPairs P, DMeshes M, DBodie
             base[threadIdx.x] = pre[threadIdx.x] + atomicAdd(&bucket_cur[threadIdx.x], h[threadIdx.x]);
         __syncthreads();
         if (p < n) {
-            if (tz) {
-                // the topology's per-pair outputs start at zero (k_topo_zero)
-                T.ncontrib[p] = 0;
-                T.comps[p] = 0;
-                T.loops_raw[p] = 0;
-                T.tstatus[p] = 0;
-                if (cur_active) cur_active[p] = 0;
-            }
+            if (tz) topo_zero_pair(T, cur_active, p);
             const int slot = base[b] + r;
             order[slot] = p;
             make_item(P, M, B, p, slot);
@@ -1594,13 +1768,8 @@ __global__ void __launch_bounds__(64, WPS) k_tp_walk_bcd_sim(DPairs P, DMeshes M
 __global__ void k_topo_zero(DPairs P, TopoBufs T, uint8_t* cur_active, unsigned long long* stamp) {
     stamp_here(stamp);
     const int n = *P.n;
-    for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x) {
-        T.ncontrib[p] = 0;
-        T.comps[p] = 0;
-        T.loops_raw[p] = 0;
-        T.tstatus[p] = 0;
-        if (cur_active) cur_active[p] = 0;
-    }
+    for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x)
+        topo_zero_pair(T, cur_active, p);
 }
 
 struct ApiSink {
@@ -2156,6 +2325,10 @@ void launch_broadphase(const BroadPhaseBufs& bp, hipStream_t s, const NeedLists*
     StepZero sz{};
     if (kt0 && z) sz = *z;
     const int n = bp.n;
+    if (n <= BP_SMALL) {
+        hipLaunchKernelGGL(k_bp_small, dim3(1), dim3(1024), 0, s, bp, nl, z ? kt0 : nullptr, sz);
+        return;
+    }
     hipLaunchKernelGGL(k_bp_bounds_part, dim3(BP_PARTS), dim3(256), 0, s, bp.state, bp.radius, n, bp.part,
                        z ? kt0 : nullptr, sz);
     // k_bp_cells writes the grid and its cell count (to a scalar, n_adj,
@@ -2183,9 +2356,9 @@ static void launch_pairs(const DBodies& B, const DMeshes& M, const DPairs& P, co
                          unsigned int* q, hipStream_t s, int wave_groups, int32_t wave_tests,
                          unsigned long long* stamp) {
     // without the work ordering (plain mode) the items in pair order
-    if (!P.order) {
+    if (!P.order && !cfg.items_made) {
         hipLaunchKernelGGL(k_pair_items, dim3(std::max(1, std::min(nblk(P.cap, 256), 1024))), dim3(256), 0, s, P, M, B,
-                           stamp);
+                           TopoBufs{}, (uint8_t*)nullptr, 0, stamp);
         stamp = nullptr;
     }
     auto group = [&](auto kernel, int bs, int back, hipStream_t gs) {
@@ -2298,6 +2471,12 @@ void launch_lpt_order(const DPairs& P, const DMeshes& M, const DBodies& B, int32
     hipLaunchKernelGGL(k_lpt_count, dim3(g), dim3(256), 0, s, P, M, B, bcnt, stamp);
     hipLaunchKernelGGL(k_lpt_scatter, dim3(g), dim3(256), 0, s, P, M, B, (const int32_t*)bcnt, bcur, order, T,
                        tz ? cur_active : nullptr, tz ? 1 : 0);
+}
+
+void launch_pair_items(const DPairs& P, const DMeshes& M, const DBodies& B, const TopoBufs& T, uint8_t* cur_active,
+                       hipStream_t s, unsigned long long* stamp) {
+    hipLaunchKernelGGL(k_pair_items, dim3(std::max(1, std::min(nblk(P.cap, 256), 1024))), dim3(256), 0, s, P, M, B, T,
+                       cur_active, 1, stamp);
 }
 
 void launch_topo_zero(const DPairs& P, const TopoBufs& T, uint8_t* cur_active, int32_t pair_cap, hipStream_t s,
