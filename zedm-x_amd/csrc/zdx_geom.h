@@ -489,6 +489,21 @@ ZDX_HD inline void basis(const V3& n, V3& u, V3& v) {
     v = cross(n, u);
 }
 
+ZDX_HD inline int popc64(uint64_t m) { return __builtin_popcountll(m); }
+// The sum of f(m), m = 0..n-1, in that order: the terms lane-parallel, added
+// one after the other by every lane.
+template <class WP, class F>
+ZDX_HD inline double ordered_sum(const WP& wp, int n, F&& f) {
+    double a = 0.0;
+    for (int mb = 0; mb < n; mb += WP::W) {
+        const int m = mb + wp.lane();
+        const double t = f(m < n ? m : n - 1);
+        const int c = n - mb < WP::W ? n - mb : WP::W;
+        for (int l = 0; l < c; ++l) a += wp.shfl(t, l);
+    }
+    return a;
+}
+
 // compute_wall_contact main.cpp:1205-1258 for one wall triangle, run by the
 // W lanes of a lane policy: the particle's world vertices are already
 // computed (the reference re-transforms the mesh per wall triangle;
@@ -497,24 +512,29 @@ ZDX_HD inline void basis(const V3& n, V3& u, V3& v) {
 // 1172-1201) tests the (triangle, edge) slots lane-parallel; crossings are
 // taken in slot order from the ballot mask and kept unless an earlier kept
 // point lies within tol (unique_points 561-577), the kept-list check again
-// lane-parallel.  Clip, area and centroid run redundantly on every lane.
+// lane-parallel.  The clip's decision for an edge needs only its two ends, so
+// it is lane-parallel too, with the outputs' places from ballots; the area's
+// and centroid's terms are added in the reference's order.
 // wv: world vertex array (3 doubles each); tri: vertex indices (3 per tri).
+// V: the number of world vertices (every triangle corner is one of them).
+// dist (optional, V doubles): the vertices' signed distances, computed once
+// instead of at every slot.
 // Scratch (shared by the lanes): pts (3 cap_pts doubles), poly buffers A/B
 // (2 (cap_pts + 8) doubles each).
-// V: the number of world vertices (every triangle corner is one of them).
 // srcs (optional, cap_pts entries): the (triangle, edge) slot 3 t + e each
 // kept section point came from, for wall_contact_jac.
 template <class WP>
 ZDX_HD inline bool wall_contact(const WP& wp, const double* wv, const int* tri, int T, int V, const V3* wt,
-                                const V3& wn, double tol, SArr<double> pts, SArr<double> PA, SArr<double> PB,
+                                const V3& wn, double tol, double* dist, double* pts, double* PA, double* PB,
                                 int cap_pts, double& area_out, V3& xc_out, V3& n_out, int& status,
                                 int32_t* srcs = nullptr) {
-    const int W = WP::W;
+    constexpr int W = WP::W;
     const int ln = wp.lane();
     V3 pn = wn;
     double pd = -dot(pn, wt[0]);
     const double t2 = tol * tol;
     int np = 0;
+    wp.sync();   // the scratch is rewritten
     // An edge crosses the plane only when its endpoints' signed distances
     // (computed below exactly as here) have a negative product, so only when
     // some vertex lies strictly below and some strictly above: without both,
@@ -525,104 +545,123 @@ ZDX_HD inline bool wall_contact(const WP& wp, const double* wv, const int* tri, 
             const int v = vb + ln;
             if (v < V) {
                 const double d = dot(pn, v3(wv[3 * v], wv[3 * v + 1], wv[3 * v + 2])) + pd;
+                if (dist) dist[v] = d;
                 below = below || d < 0.0;
                 above = above || d > 0.0;
             }
-            if (wp.ballot(below) != 0ull && wp.ballot(above) != 0ull) break;
+            if (!dist && wp.ballot(below) != 0ull && wp.ballot(above) != 0ull) break;
         }
         if (!(wp.ballot(below) != 0ull && wp.ballot(above) != 0ull)) return false;
+        wp.sync();
     }
     const int nslots = 3 * T;
-    for (int base = 0; base < nslots; base += W) {
-        const int f = base + ln;
-        bool hit = false;
-        V3 ip = v3(0.0, 0.0, 0.0);
-        if (f < nslots) {
-            const int t = f / 3, i = f - 3 * t;
-            const int i0 = tri[3 * t + i], i1 = tri[3 * t + (i + 1) % 3];
-            V3 p0 = v3(wv[3 * i0], wv[3 * i0 + 1], wv[3 * i0 + 2]);
-            V3 p1 = v3(wv[3 * i1], wv[3 * i1 + 1], wv[3 * i1 + 2]);
-            double d0 = dot(pn, p0) + pd, d1 = dot(pn, p1) + pd;
-            if (d0 * d1 < 0.0) {
-                double tt = d0 / (d0 - d1);
-                tt = dmin(1.0, dmax(0.0, tt));
-                ip = add(p0, mul(sub(p1, p0), tt));
-                hit = true;
-            }
+    constexpr int U = 2;   // rounds of slots whose loads are in flight together
+    for (int base = 0; base < nslots; base += U * W) {
+        int i0[U], i1[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int f = base + u * W + ln, t = (f < nslots ? f : 0) / 3, i = (f < nslots ? f : 0) - 3 * t;
+            i0[u] = tri[3 * t + i];
+            i1[u] = tri[3 * t + (i == 2 ? 0 : i + 1)];
         }
-        uint64_t m = wp.ballot(hit);
-        while (m) {
-            const int src = ctz64(m);
-            m &= m - 1;
-            const V3 q = v3(wp.shfl(ip.x, src), wp.shfl(ip.y, src), wp.shfl(ip.z, src));
-            bool dup = false;
-            for (int kb = 0; kb < np && !dup; kb += W) {
-                const int k = kb + ln;
-                bool near = false;
-                if (k < np) near = norm2(sub(q, v3(pts[3 * k], pts[3 * k + 1], pts[3 * k + 2]))) <= t2;
-                dup = wp.ballot(near) != 0ull;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int f = base + u * W + ln;
+            bool hit = false;
+            V3 ip = v3(0.0, 0.0, 0.0);
+            if (f < nslots) {
+                const double* a = wv + 3 * i0[u];
+                const double* b = wv + 3 * i1[u];
+                double d0, d1;
+                if (dist) {
+                    d0 = dist[i0[u]]; d1 = dist[i1[u]];
+                } else {
+                    d0 = dot(pn, v3(a[0], a[1], a[2])) + pd; d1 = dot(pn, v3(b[0], b[1], b[2])) + pd;
+                }
+                if (d0 * d1 < 0.0) {
+                    const V3 p0 = v3(a[0], a[1], a[2]), p1 = v3(b[0], b[1], b[2]);
+                    double tt = d0 / (d0 - d1);
+                    tt = dmin(1.0, dmax(0.0, tt));
+                    ip = add(p0, mul(sub(p1, p0), tt));
+                    hit = true;
+                }
             }
-            if (!dup) {
-                if (np >= cap_pts) { status = 1; return false; }
-                pts[3 * np] = q.x; pts[3 * np + 1] = q.y; pts[3 * np + 2] = q.z;
-                if (srcs) srcs[np] = base + src;
-                ++np;
+            uint64_t m = wp.ballot(hit);
+            while (m) {
+                const int src = ctz64(m);
+                m &= m - 1;
+                const V3 q = v3(wp.shfl(ip.x, src), wp.shfl(ip.y, src), wp.shfl(ip.z, src));
+                bool dup = false;
+                for (int kb = 0; kb < np && !dup; kb += W) {
+                    const int k = kb + ln;
+                    bool near = false;
+                    if (k < np) near = norm2(sub(q, v3(pts[3 * k], pts[3 * k + 1], pts[3 * k + 2]))) <= t2;
+                    dup = wp.ballot(near) != 0ull;
+                }
+                if (!dup) {
+                    if (np >= cap_pts) { status = 1; return false; }
+                    pts[3 * np] = q.x; pts[3 * np + 1] = q.y; pts[3 * np + 2] = q.z;
+                    if (srcs) srcs[np] = base + u * W + src;
+                    ++np;
+                }
             }
         }
     }
     if (srcs) srcs[cap_pts] = np;   // the count, after the slots
     if (np < 3) return false;
+    wp.sync();
     V3 bu, bv;
     basis(pn, bu, bv);
     V3 o = wt[0];
-    for (int m = 0; m < np; ++m) {
+    for (int m = ln; m < np; m += W) {
         V3 d = sub(v3(pts[3 * m], pts[3 * m + 1], pts[3 * m + 2]), o);
         PA[2 * m] = dot(d, bu);
         PA[2 * m + 1] = dot(d, bv);
     }
     V2 clip[3];
     for (int k = 0; k < 3; ++k) { V3 d = sub(wt[k], o); clip[k] = v2(dot(d, bu), dot(d, bv)); }
-    // sutherland_hodgman_clip 1093-1122
+    // sutherland_hodgman_clip 1093-1122: an edge (sv, e) gives its crossing
+    // with the clip line where exactly one end is inside, then e if it is
+    const uint64_t below = (1ull << ln) - 1ull;
     int nin = np;
-    SArr<double> in = PA, outp = PB;
+    double *in = PA, *outp = PB;
     V2 c1 = clip[2];
     for (int ck = 0; ck < 3; ++ck) {
         V2 c2 = clip[ck];
         if (nin == 0) break;
         int nout = 0;
-        V2 sv = v2(in[2 * (nin - 1)], in[2 * (nin - 1) + 1]);
-        for (int m = 0; m < nin; ++m) {
-            V2 e = v2(in[2 * m], in[2 * m + 1]);
-            if (inside_clip(e, c1, c2)) {
-                if (!inside_clip(sv, c1, c2)) {
-                    V2 x = isect_clip(sv, e, c1, c2);
-                    if (nout >= cap_pts + 6) { status = 1; return false; }
-                    outp[2 * nout] = x.x; outp[2 * nout + 1] = x.y; ++nout;
-                }
-                if (nout >= cap_pts + 6) { status = 1; return false; }
-                outp[2 * nout] = e.x; outp[2 * nout + 1] = e.y; ++nout;
-            } else if (inside_clip(sv, c1, c2)) {
-                V2 x = isect_clip(sv, e, c1, c2);
-                if (nout >= cap_pts + 6) { status = 1; return false; }
-                outp[2 * nout] = x.x; outp[2 * nout + 1] = x.y; ++nout;
+        wp.sync();
+        for (int mb = 0; mb < nin; mb += W) {
+            const int m = mb + ln, mi = m < nin ? m : nin - 1, ms = mi > 0 ? mi - 1 : nin - 1;
+            const V2 e = v2(in[2 * mi], in[2 * mi + 1]), sv = v2(in[2 * ms], in[2 * ms + 1]);
+            const bool ein = inside_clip(e, c1, c2), sin_ = inside_clip(sv, c1, c2);
+            const bool cross_ = m < nin && ein != sin_, keep = m < nin && ein;
+            const uint64_t bc = wp.ballot(cross_), bk = wp.ballot(keep);
+            int at = nout + popc64(bc & below) + popc64(bk & below);
+            if (cross_) {
+                const V2 x = isect_clip(sv, e, c1, c2);
+                if (at < cap_pts + 6) { outp[2 * at] = x.x; outp[2 * at + 1] = x.y; }
+                ++at;
             }
-            sv = e;
+            if (keep && at < cap_pts + 6) { outp[2 * at] = e.x; outp[2 * at + 1] = e.y; }
+            nout += popc64(bc) + popc64(bk);
         }
-        SArr<double> tmp = in; in = outp; outp = tmp;
+        if (nout > cap_pts + 6) { status = 1; return false; }
+        double* tmp = in; in = outp; outp = tmp;
         nin = nout;
         c1 = c2;
     }
     if (nin < 3) return false;
+    wp.sync();
     // polygon_area_2d / polygon_centroid_2d 1125-1146
-    double a = 0.0;
-    for (int m = 0; m < nin; ++m) {
-        int j = (m + 1) % nin;
-        a += cr2(v2(in[2 * m], in[2 * m + 1]), v2(in[2 * j], in[2 * j + 1]));
-    }
+    double a = ordered_sum(wp, nin, [&](int m) {
+        const int j = m + 1 < nin ? m + 1 : 0;
+        return cr2(v2(in[2 * m], in[2 * m + 1]), v2(in[2 * j], in[2 * j + 1]));
+    });
     a = fabs(a) * 0.5;
     if (a < tol * tol * 0.01) return false;
-    double cx = 0.0, cy = 0.0;
-    for (int m = 0; m < nin; ++m) { cx += in[2 * m]; cy += in[2 * m + 1]; }
+    const double cx = ordered_sum(wp, nin, [&](int m) { return in[2 * m]; });
+    const double cy = ordered_sum(wp, nin, [&](int m) { return in[2 * m + 1]; });
     double nn = (double)nin;
     V2 c = v2(cx / nn, cy / nn);
     area_out = a;
@@ -633,7 +672,7 @@ ZDX_HD inline bool wall_contact(const WP& wp, const double* wv, const int* tri, 
 
 // Derivatives of a wall contact (area and contact point of wall_contact)
 // with respect to a rigid motion xi = (d, w) of the particle: every world
-// vertex p moves by d + w x (p - x).  One thread; it repeats wall_contact's
+// vertex p moves by d + w x (p - x).  The lanes repeat wall_contact's
 // arithmetic on the kept section points (srcs: their edge slots and count,
 // as wall_contact recorded them) with six tangents carried beside each value,
 // so every branch (clip tests, area sign) is decided on the same doubles.
@@ -641,11 +680,15 @@ ZDX_HD inline bool wall_contact(const WP& wp, const double* wv, const int* tri, 
 // p1) with signed distances d0, d1 to the wall plane, has the tangent
 // dp0 + t (dp1 - dp0) + (p1 - p0) dt, dt = (d0 dd1 - d1 dd0) / (d0 - d1)^2.
 // Scratch T: 14 (cap_pts + 8) doubles per polygon buffer, two buffers.
-// dA: 6 doubles; dX: 3 x 6 (row-major).  Returns false when wall_contact
-// would (no contact).
-ZDX_HD inline bool wall_contact_jac(const double* wv, const int* tri, const V3& x, const V3* wt, const V3& wn,
-                                    double tol, const int32_t* srcs, int cap_pts, SArr<double> TA, SArr<double> TB,
+// dA: 6 doubles; dX: 3 x 6 (row-major), in every lane.  Returns false when
+// wall_contact would (no contact).
+template <class WP>
+ZDX_HD inline bool wall_contact_jac(const WP& wp, const double* wv, const int* tri, const V3& x, const V3* wt,
+                                    const V3& wn, double tol, const int32_t* srcs, int cap_pts, double* TA, double* TB,
                                     double* dA, double* dX) {
+    constexpr int W = WP::W;
+    const int ln = wp.lane();
+    wp.sync();
     const int np = srcs[cap_pts];
     if (np < 3) return false;
     V3 pn = wn;
@@ -654,7 +697,7 @@ ZDX_HD inline bool wall_contact_jac(const double* wv, const int* tri, const V3& 
     basis(pn, bu, bv);
     V3 o = wt[0];
     // polygon vertex m: [0] u, [1] v, [2..8) du/dxi, [8..14) dv/dxi
-    for (int m = 0; m < np; ++m) {
+    for (int m = ln; m < np; m += W) {
         const int f = srcs[m];
         const int t = f / 3, i = f - 3 * t;
         const int i0 = tri[3 * t + i], i1 = tri[3 * t + (i + 1) % 3];
@@ -683,76 +726,74 @@ ZDX_HD inline bool wall_contact_jac(const double* wv, const int* tri, const V3& 
     V2 clip[3];
     for (int k = 0; k < 3; ++k) { V3 d = sub(wt[k], o); clip[k] = v2(dot(d, bu), dot(d, bv)); }
     // sutherland_hodgman_clip 1093-1122 with tangents
+    const uint64_t below = (1ull << ln) - 1ull;
     int nin = np;
-    SArr<double> in = TA, outp = TB;
+    double *in = TA, *outp = TB;
     V2 c1 = clip[2];
-    auto emit = [&](int& nout, const double* src14) {
-        for (int q = 0; q < 14; ++q) outp[14 * nout + q] = src14[q];
-        ++nout;
-    };
     for (int ck = 0; ck < 3; ++ck) {
         V2 c2 = clip[ck];
         if (nin == 0) break;
         int nout = 0;
-        int sidx = nin - 1;
-        for (int m = 0; m < nin; ++m) {
-            V2 e = v2(in[14 * m], in[14 * m + 1]);
-            V2 sv = v2(in[14 * sidx], in[14 * sidx + 1]);
+        wp.sync();
+        for (int mb = 0; mb < nin; mb += W) {
+            const int m = mb + ln, mi = m < nin ? m : nin - 1, ms = mi > 0 ? mi - 1 : nin - 1;
+            const double *pe = in + 14 * mi, *ps = in + 14 * ms;
+            const V2 e = v2(pe[0], pe[1]), sv = v2(ps[0], ps[1]);
             const bool ein = inside_clip(e, c1, c2), sin_ = inside_clip(sv, c1, c2);
-            if (ein != sin_) {
+            const bool cross_ = m < nin && ein != sin_, keep = m < nin && ein;
+            const uint64_t bc = wp.ballot(cross_), bk = wp.ballot(keep);
+            int at = nout + popc64(bc & below) + popc64(bk & below);
+            if (cross_) {
                 // the crossing of the edge (sv, e) with the clip line
-                double rec[14];
+                double* q = outp + 14 * at;
                 V2 dc = sub2(c1, c2), dp = sub2(sv, e);
                 double n1 = cr2(c1, c2), n2 = cr2(sv, e), n3 = cr2(dc, dp);
-                if (fabs(n3) < 1e-30) {
-                    for (int q = 0; q < 14; ++q) rec[q] = in[14 * sidx + q];
+                if (at >= cap_pts + 6) {
+                } else if (fabs(n3) < 1e-30) {
+                    for (int k = 0; k < 14; ++k) q[k] = ps[k];
                 } else {
                     const double X = (n1 * dp.x - n2 * dc.x) / n3, Y = (n1 * dp.y - n2 * dc.y) / n3;
-                    rec[0] = X;
-                    rec[1] = Y;
+                    q[0] = X;
+                    q[1] = Y;
                     for (int j = 0; j < 6; ++j) {
-                        V2 dsv = v2(in[14 * sidx + 2 + j], in[14 * sidx + 8 + j]);
-                        V2 de = v2(in[14 * m + 2 + j], in[14 * m + 8 + j]);
+                        V2 dsv = v2(ps[2 + j], ps[8 + j]);
+                        V2 de = v2(pe[2 + j], pe[8 + j]);
                         V2 ddp = sub2(dsv, de);
                         const double dn2 = cr2(dsv, e) + cr2(sv, de), dn3 = cr2(dc, ddp);
-                        rec[2 + j] = (n1 * ddp.x - dn2 * dc.x - X * dn3) / n3;
-                        rec[8 + j] = (n1 * ddp.y - dn2 * dc.y - Y * dn3) / n3;
+                        q[2 + j] = (n1 * ddp.x - dn2 * dc.x - X * dn3) / n3;
+                        q[8 + j] = (n1 * ddp.y - dn2 * dc.y - Y * dn3) / n3;
                     }
                 }
-                if (nout >= cap_pts + 6) return false;
-                emit(nout, rec);
+                ++at;
             }
-            if (ein) {
-                if (nout >= cap_pts + 6) return false;
-                double rec[14];
-                for (int q = 0; q < 14; ++q) rec[q] = in[14 * m + q];
-                emit(nout, rec);
-            }
-            sidx = m;
+            if (keep && at < cap_pts + 6)
+                for (int k = 0; k < 14; ++k) outp[14 * at + k] = pe[k];
+            nout += popc64(bc) + popc64(bk);
         }
-        SArr<double> tmp = in; in = outp; outp = tmp;
+        if (nout > cap_pts + 6) return false;
+        double* tmp = in; in = outp; outp = tmp;
         nin = nout;
         c1 = c2;
     }
     if (nin < 3) return false;
-    double a = 0.0;
-    double da[6] = {0, 0, 0, 0, 0, 0};
-    for (int m = 0; m < nin; ++m) {
-        int j = (m + 1) % nin;
-        V2 pm = v2(in[14 * m], in[14 * m + 1]), pj = v2(in[14 * j], in[14 * j + 1]);
-        a += cr2(pm, pj);
-        for (int q = 0; q < 6; ++q)
-            da[q] += cr2(v2(in[14 * m + 2 + q], in[14 * m + 8 + q]), pj) +
-                     cr2(pm, v2(in[14 * j + 2 + q], in[14 * j + 8 + q]));
-    }
+    wp.sync();
+    auto next = [&](int m) { return m + 1 < nin ? m + 1 : 0; };
+    double a = ordered_sum(wp, nin, [&](int m) {
+        const double *pm = in + 14 * m, *pj = in + 14 * next(m);
+        return cr2(v2(pm[0], pm[1]), v2(pj[0], pj[1]));
+    });
     const double sg = a < 0.0 ? -0.5 : 0.5;
     a = fabs(a) * 0.5;
     if (a < tol * tol * 0.01) return false;
     const double nn = (double)nin;
     for (int q = 0; q < 6; ++q) {
-        double su = 0.0, sv2 = 0.0;
-        for (int m = 0; m < nin; ++m) { su += in[14 * m + 2 + q]; sv2 += in[14 * m + 8 + q]; }
-        dA[q] = sg * da[q];
+        const double da = ordered_sum(wp, nin, [&](int m) {
+            const double *pm = in + 14 * m, *pj = in + 14 * next(m);
+            return cr2(v2(pm[2 + q], pm[8 + q]), v2(pj[0], pj[1])) + cr2(v2(pm[0], pm[1]), v2(pj[2 + q], pj[8 + q]));
+        });
+        const double su = ordered_sum(wp, nin, [&](int m) { return in[14 * m + 2 + q]; });
+        const double sv2 = ordered_sum(wp, nin, [&](int m) { return in[14 * m + 8 + q]; });
+        dA[q] = sg * da;
         V3 dxq = add(mul(bu, su / nn), mul(bv, sv2 / nn));
         dX[q] = dxq.x; dX[6 + q] = dxq.y; dX[12 + q] = dxq.z;
     }

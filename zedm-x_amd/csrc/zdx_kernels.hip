@@ -1851,35 +1851,34 @@ __device__ inline bool wall_tri_candidate(const double* wt9, const V3& pmn, cons
 
 // One wave per listed particle (a particle near at least one wall triangle).
 // Entries of particles not in the list were zeroed before this kernel.
-// Registers capped at 96 (five waves per SIMD): the kernel runs beside the
-// narrow phase on the second stream, and at its natural 206 VGPRs a walls wave
-// left room for only two of the one-wave narrow kernel's waves on its SIMD
-// instead of four (the narrow phase is 3 % faster this way; the walls, which
-// end well before it, spill a little).
-__global__ void __launch_bounds__(64, 5) k_walls(DBodies B, DMeshes M, DMat mat, WallBufs W, HistBufs H, double* wcontrib,
+// Registers capped at 128 (four waves per SIMD) and no LDS: the kernel runs
+// beside the narrow phase on the second stream, whose one-wave-per-pair kernel
+// fills a CU's LDS.  In the 60k packing 917 us (three waves 811, five 948; 968
+// before the clip and the slots' loads were spread over the lanes) beside 850
+// us of that kernel; with the distances and the section in 9 KB of LDS 774 us,
+// but that kernel then took 1150.
+__global__ void __launch_bounds__(64, 4) k_walls(DBodies B, DMeshes M, DMat mat, WallBufs W, HistBufs H, double* wcontrib,
                                               int32_t* wnc, const int32_t* list, const int32_t* n_list, double* scr,
                                               int32_t pts_cap, SimParams sp, int32_t* status) {
     LaneDev wp;
     const int nl = *n_list;
     const int64_t per = 3 * (int64_t)pts_cap + 4 * (int64_t)(pts_cap + 8);
-    SArr<double> PTS; PTS.p = scr + (int64_t)blockIdx.x * per; PTS.s = 1;
-    SArr<double> PA = PTS.at(3 * (int64_t)pts_cap);
-    SArr<double> PB = PA.at(2 * (int64_t)(pts_cap + 8));
+    double* PTS = scr + (int64_t)blockIdx.x * per;
+    double *PA = PTS + 3 * (int64_t)pts_cap, *PB = PA + 2 * (int64_t)(pts_cap + 8);
     for (int it = blockIdx.x; it < nl; it += gridDim.x) {
         const int i = list[it];
-        Body p = load_body(B.state + 16 * (int64_t)i);
+        const V3 pos = ld3(B.state + 16 * (int64_t)i);
         const double r = mat.radius[i];
         const int m = B.mesh[i];
         const double tol = M.tol[m];
         const double* wv = B.wv + 3 * B.wv_off[i];
         const int32_t* ti = M.tri_idx + 3 * (int64_t)M.tri_off[m];
         const int T = M.ntris[m];
-        Mat mt = load_mat(mat, i);
-        V3 pmn = sub(p.pos, v3(r, r, r)), pmx = add(p.pos, v3(r, r, r));
+        V3 pmn = sub(pos, v3(r, r, r)), pmx = add(pos, v3(r, r, r));
         for (int w = 0; w < W.n_walls; ++w) {
             const int64_t idx = (int64_t)i * W.n_walls + w;
             // sphere test main.cpp:2318-2323
-            V3 dp = sub(p.pos, ld3(W.pos + 3 * w));
+            V3 dp = sub(pos, ld3(W.pos + 3 * w));
             double d2 = dot(dp, dp);
             double rs = r + W.radius[w];
             int nc = 0;
@@ -1893,13 +1892,15 @@ __global__ void __launch_bounds__(64, 5) k_walls(DBodies B, DMeshes M, DMat mat,
                     double area;
                     V3 xc, cn;
                     int st = 0;
-                    bool ok = wall_contact(wp, wv, ti, T, M.nverts[m], wt, ld3(W.normals + 3 * (int64_t)(t0 + t)), tol, PTS, PA,
-                                           PB, pts_cap, area, xc, cn, st);
+                    const bool ok = wall_contact(wp, wv, ti, T, M.nverts[m], wt, ld3(W.normals + 3 * (int64_t)(t0 + t)),
+                                                 tol, nullptr, PTS, PA, PB, pts_cap, area, xc, cn, st);
                     if (!ok) {
                         if (st && lane_id() == 0) atomicOr(status, (int)ST_WALL);
                         continue;
                     }
-                    Contact c = pw_force(cn, area, xc, p, mt, W.mu[w], sp.dt, ds);
+                    // the body and its material are read here, not held across the section
+                    Contact c = pw_force(cn, area, xc, load_body(B.state + 16 * (int64_t)i), load_mat(mat, i), W.mu[w],
+                                         sp.dt, ds);
                     if (nc < W.max_wall_tris && lane_id() == 0) {
                         double* o = wcontrib + 6 * (idx * W.max_wall_tris + nc);
                         o[0] = c.f.x; o[1] = c.f.y; o[2] = c.f.z; o[3] = c.r1.x; o[4] = c.r1.y; o[5] = c.r1.z;
@@ -2207,48 +2208,66 @@ __global__ void __launch_bounds__(256) k_copy_parts(CopyParts k) {
     if (at == 0 && k.zero) *k.zero = 0;
 }
 
+// One wave per (body, wall triangle), its scratch in LDS (40 KB, four per CU)
+// when mesh and section fit there.  It is bound by the latency of one wave's
+// chain; 61 bodies against 12 triangles with Jacobians took 179 us with one
+// lane clipping and carrying the tangents through global memory, the whole call
+// 229 us then and 112 so.
 __global__ void __launch_bounds__(64) k_wall_query(DBodies B, DMeshes M, int32_t n_bodies, const double* tris,
                                                    const double* normals, int32_t n_tris, int32_t jac, int32_t cap,
                                                    double* scr, int32_t* isrc, double* out, int32_t* status) {
+    constexpr int LV = 1280, LP = 96;   // vertices and section points held in LDS
+    __shared__ double s_d[LV], s_p[3 * LP + 4 * (LP + 8)], s_t[28 * (LP + 8)];
+    __shared__ int32_t s_src[LP + 1];
     LaneDev wp;
     const int64_t q = blockIdx.x;
     if (q >= (int64_t)n_bodies * n_tris) return;
     const int b = (int)(q / n_tris), t = (int)(q - (int64_t)b * n_tris);
-    const int64_t per = 3 * (int64_t)cap + 4 * (int64_t)(cap + 8) + 28 * (int64_t)(cap + 8);
-    SArr<double> PTS; PTS.p = scr + q * per; PTS.s = 1;
-    SArr<double> PA = PTS.at(3 * (int64_t)cap);
-    SArr<double> PB = PA.at(2 * (int64_t)(cap + 8));
-    SArr<double> TA = PB.at(2 * (int64_t)(cap + 8));
-    SArr<double> TB = TA.at(14 * (int64_t)(cap + 8));
-    int32_t* src = isrc + q * (int64_t)(cap + 1);
     const int m = B.mesh[b];
     const double* wv = B.wv + 3 * B.wv_off[b];
     const int32_t* ti = M.tri_idx + 3 * (int64_t)M.tri_off[m];
     const double* wt9 = tris + 9 * (int64_t)t;
     V3 wt[3] = {ld3(wt9), ld3(wt9 + 3), ld3(wt9 + 6)};
     const V3 wn = ld3(normals + 3 * (int64_t)t);
-    double area = 0.0;
+    const Body p = load_body(B.state + 16 * (int64_t)b);
+    const int T = M.ntris[m], V = M.nverts[m];
+    const double tol = M.tol[m];
+    double area = 0.0, o[32], dA[6], dX[18];
     V3 xc, cn;
     int st = 0;
-    const bool ok = wall_contact(wp, wv, ti, M.ntris[m], M.nverts[m], wt, wn, M.tol[m], PTS, PA, PB, cap, area, xc,
-                                 cn, st, src);
-    double* o = out + 32 * q;
-    if (lane_id() != 0) return;
-    for (int k = 0; k < 32; ++k) o[k] = 0.0;
-    if (!ok) {
-        if (st) atomicOr(status, 1);
-        return;
+    bool same = true;
+    const int lp = cap < LP ? cap : LP;
+    bool ok = false;
+    if (V <= LV)
+        ok = wall_contact(wp, wv, ti, T, V, wt, wn, tol, s_d, s_p, s_p + 3 * LP, s_p + 3 * LP + 2 * (LP + 8), lp, area, xc,
+                          cn, st, s_src);
+    if (ok && jac)
+        same = wall_contact_jac(wp, wv, ti, p.pos, wt, wn, tol, s_src, lp, s_t, s_t + 14 * (LP + 8), dA, dX);
+    if (V > LV || (st && cap > lp)) {   // more than the LDS holds
+        const int64_t per = 3 * (int64_t)cap + 32 * (int64_t)(cap + 8);
+        double* PTS = scr + q * per;
+        double *PA = PTS + 3 * (int64_t)cap, *PB = PA + 2 * (int64_t)(cap + 8), *TA = PB + 2 * (int64_t)(cap + 8);
+        int32_t* src = isrc + q * (int64_t)(cap + 1);
+        st = 0;
+        ok = wall_contact(wp, wv, ti, T, V, wt, wn, tol, nullptr, PTS, PA, PB, cap, area, xc, cn, st, src);
+        if (ok && jac)
+            same = wall_contact_jac(wp, wv, ti, p.pos, wt, wn, tol, src, cap, TA, TA + 14 * (int64_t)(cap + 8), dA, dX);
     }
-    const Body p = load_body(B.state + 16 * (int64_t)b);
-    if (dot(cn, sub(p.pos, xc)) < 0.0) cn = mul(cn, -1.0);   // main.cpp:2363-2367
-    o[0] = 1.0; o[1] = area;
-    o[2] = xc.x; o[3] = xc.y; o[4] = xc.z;
-    o[5] = cn.x; o[6] = cn.y; o[7] = cn.z;
-    if (jac) {
-        if (!wall_contact_jac(wv, ti, p.pos, wt, wn, M.tol[m], src, cap, TA, TB, o + 8, o + 14)) {
-            atomicOr(status, 2);   // cannot differ from wall_contact: same doubles, same branches
+    for (int k = 0; k < 32; ++k) o[k] = 0.0;
+    if (ok) {
+        if (dot(cn, sub(p.pos, xc)) < 0.0) cn = mul(cn, -1.0);   // main.cpp:2363-2367
+        o[0] = 1.0; o[1] = area;
+        o[2] = xc.x; o[3] = xc.y; o[4] = xc.z;
+        o[5] = cn.x; o[6] = cn.y; o[7] = cn.z;
+        if (jac && same) {
+            for (int k = 0; k < 6; ++k) o[8 + k] = dA[k];
+            for (int k = 0; k < 18; ++k) o[14 + k] = dX[k];
         }
     }
+    if (lane_id() != 0) return;
+    for (int k = 0; k < 32; ++k) out[32 * q + k] = o[k];
+    if (!ok && st) atomicOr(status, 1);
+    if (ok && jac && !same) atomicOr(status, 2);   // cannot differ from wall_contact: same doubles, same branches
 }
 
 __global__ void k_or_i32(const int32_t* v, int32_t n, int32_t* out) {
