@@ -1536,16 +1536,6 @@ __device__ inline WalkB tp_walk_b_item(const DPairs& P, const DMeshes& M, const 
     return WalkB{ncomp, ncomp >= 0 ? to : -1};
 }
 
-// Walk B: components, snapped vertices and edges of each pair; allocates the
-// pair's T-junction words.  The adjacency rows are copied into the scratch.
-__global__ void __launch_bounds__(64) k_tp_walk_b(DPairs P, DMeshes M, DBodies B, TopoBufs T, int32_t split,
-                                                  int32_t lds_bytes) {
-    extern __shared__ char s_walk[];
-    const int n = *P.topo_n;
-    LaneDev wp;
-    for (int it = blockIdx.x; it < n; it += gridDim.x) tp_walk_b_item(P, M, B, T, split, lds_bytes, s_walk, wp, it);
-}
-
 // Pass C: T-junction hit words of every component of an item; each wave of
 // the workgroup covers 64 vertices of one edge row per ballot.
 // lds / lds_bytes (optional): a component's vertices, cells and edges are
@@ -1620,11 +1610,6 @@ __device__ inline void tp_pass_c_item(const DPairs& P, const DMeshes& M, const D
         __syncthreads();   // the staged component is replaced by the next one
     }
 }
-__global__ void __launch_bounds__(256) k_tp_pass_c(DPairs P, DMeshes M, DBodies B, TopoBufs T) {
-    const int n = *P.topo_n;
-    for (int it = blockIdx.x; it < n; it += gridDim.x) tp_pass_c_item(P, M, B, T, it, T.ncomp[it], T.tj_off[it]);
-}
-
 // Walk D with its inputs copied to the scratch: edges, vertex cells.
 template <class Sink, bool SENS = true>
 __device__ inline TopoOut tp_walk_d(const LaneDev& wp, const TopoBufs& T, int S, int ncomp, int64_t sb, long long to,
@@ -1810,11 +1795,22 @@ struct ApiSink {
     static constexpr int ZDX_LOOP_REC_D = 28;
 };
 
-__global__ void __launch_bounds__(64) k_tp_walk_d_api(DPairs P, DMeshes M, DBodies B, TopoBufs T, int32_t lds_bytes) {
+// Walk B, pass C and walk D of one item in a row on one wave, as the time step
+// runs them: a pair does not wait for the slowest of each stage.  4096 pairs of
+// about 80 segments: the whole call 1755 us with a launch per stage (220, 133
+// and 358 us), 1660 so; registers for two waves per SIMD give the same there and
+// cost 257 pairs with sensitivities 6 %.
+template <bool SENS>
+__global__ void __launch_bounds__(64, 1) k_tp_walk_bcd_api(DPairs P, DMeshes M, DBodies B, TopoBufs T,
+                                                           int32_t split, int32_t lds_bytes) {
     extern __shared__ char s_walk[];
     const int n = *P.topo_n;
     LaneDev wp;
     for (int it = blockIdx.x; it < n; it += gridDim.x) {
+        const WalkB r = tp_walk_b_item<SENS>(P, M, B, T, split, lds_bytes, s_walk, wp, it);
+        __syncthreads();
+        tp_pass_c_item(P, M, B, T, it, r.ncomp, r.to, s_walk, lds_bytes);
+        __syncthreads();
         const int p = P.topo_list[it];
         const int i = P.pi[p], j = P.pj[p];
         const int S = P.nseg[p];
@@ -1822,14 +1818,12 @@ __global__ void __launch_bounds__(64) k_tp_walk_d_api(DPairs P, DMeshes M, DBodi
         const V3 pa = ld3(B.state + 16 * (int64_t)i), pb = ld3(B.state + 16 * (int64_t)j);
         ApiSink sink{T.rec + 28 * (int64_t)p * T.lmax, T.vtx ? T.vtx + 3 * (int64_t)p * T.vmax : nullptr,
                      T.lmax, T.vmax, 0, pa, pb, T.k_stiff, T.ljac ? T.ljac + 72 * (int64_t)p * T.lmax : nullptr};
-        const int ncomp = T.ncomp[it];
-        const long long to = T.tj_off[it];
         TopoOut o;
         o.comps = 0; o.loops_raw = 0; o.loops = 0; o.status = 0;
-        if (ncomp < 0 || to < 0) o.status = TOPO_E2_OVERFLOW;
-        else if (ncomp > 0)
-            o = tp_walk_d(wp, T, S, ncomp, P.seg_off[p], to, topo_tol(T, M, mA), M.area_eps[mA], sub(pb, pa), s_walk,
-                          lds_bytes, sink);
+        if (r.ncomp < 0 || r.to < 0) o.status = TOPO_E2_OVERFLOW;
+        else if (r.ncomp > 0)
+            o = tp_walk_d<ApiSink, SENS>(wp, T, S, r.ncomp, P.seg_off[p], r.to, topo_tol(T, M, mA), M.area_eps[mA],
+                                         sub(pb, pa), s_walk, lds_bytes, sink);
         if (lane_id() == 0) {
             T.ncontrib[p] = o.loops;
             T.comps[p] = o.comps;
@@ -2592,11 +2586,12 @@ void launch_topo_api(const DPairs& P, const DMeshes& M, const DBodies& B, const 
                      hipStream_t s) {
     launch_pass_a(P, M, B, T, s, true);
     if (T.ej) hipLaunchKernelGGL(k_tp_endpoint_jac, dim3((unsigned)T.pass_groups), dim3(256), 0, s, P, M, B, T);
-    hipLaunchKernelGGL(k_tp_walk_b, dim3((unsigned)T.nthreads), dim3(64), T.lds_bytes, s, P, M, B, T, split,
-                       T.lds_bytes);
-    hipLaunchKernelGGL(k_tp_pass_c, dim3((unsigned)T.pass_groups), dim3(256), 0, s, P, M, B, T);
-    hipLaunchKernelGGL(k_tp_walk_d_api, dim3((unsigned)T.nthreads), dim3(64), T.lds_bytes, s, P, M, B, T,
-                       T.lds_bytes);
+    if (T.ej)
+        hipLaunchKernelGGL(k_tp_walk_bcd_api<true>, dim3((unsigned)T.nthreads), dim3(64), T.lds_bytes, s, P, M, B, T, split,
+                           T.lds_bytes);
+    else
+        hipLaunchKernelGGL(k_tp_walk_bcd_api<false>, dim3((unsigned)T.nthreads), dim3(64), T.lds_bytes, s, P, M, B, T,
+                           split, T.lds_bytes);
 }
 void launch_walls(const DBodies& B, const DMeshes& M, const DMat& mat, const WallBufs& W, const HistBufs& H,
                   double* wcontrib, int32_t* wnc, const int32_t* list, const int32_t* n_list, double* scr,
