@@ -329,12 +329,11 @@ def _short(name):
     return name.replace("zdx::(anonymous namespace)::", "").split("(")[0].replace("void ", "")
 
 
-# the narrow phase (one launch each per step): cull + sweep with one wave per
-# pair, then a workgroup per pair for the pairs it leaves, exact tests,
-# compaction, the topology's work lists
-NARROW_KERNELS = ("k_narrow_wave", "k_narrow<", "k_narrow_exact", "k_narrow_compact", "k_topo_lists")
-NARROW_DESC = ("narrow phase: k_narrow_wave + k_narrow (cull + sweep) + k_narrow_exact + k_narrow_compact + "
-               "k_topo_lists")
+# the narrow phase (one launch each per step): clusters and box tests with one
+# wave per pair, then workgroups per pair for the two lists it leaves, exact
+# tests, ordering with the topology's work lists
+NARROW_KERNELS = ("k_pairs_",)
+NARROW_DESC = "narrow phase: k_pairs_wave + k_pairs_group (two lists, side by side) + k_pairs_exact + k_pairs_sort"
 
 
 def _is_narrow(name):

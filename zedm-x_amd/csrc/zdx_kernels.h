@@ -266,11 +266,11 @@ void launch_fold_integrate(int32_t n, const double* state_in, double* state_out,
 void launch_fill_i32(int32_t* p, int32_t v, int64_t n, hipStream_t s);
 void launch_fill_u64(unsigned long long* p, unsigned long long v, int64_t n, hipStream_t s);
 
-// Output of the per-pair call packed on the device, so that each array
-// reaches the caller in one copy: per-pair loop, vertex and segment offsets
-// (exclusive scans), then the accepted loops' records (28 doubles), their
-// Jacobians (72, optional), their vertices (optional) and the segments
-// (optional) back to back in pair order.  Optional outputs are NULL.
+// Output of the per-pair call packed on the device: per-pair loop, vertex and
+// segment offsets (exclusive scans), then the accepted loops' records (28
+// doubles), their Jacobians (72, optional), their vertices (optional) and the
+// segments (optional) back to back in pair order.
+
 // The per-pair call's host memory (pinned, one block per context): the
 // caller's pairs go to the device from its input part, small outputs come back
 // through its slots, written by the device, so that a call waits for the

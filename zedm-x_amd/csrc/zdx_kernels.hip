@@ -10,22 +10,24 @@
 //                     sort of particles by cell, per-particle neighbour
 //                     enumeration, scans, ordered pair list (i < j) and the
 //                     per-particle adjacency used by the ordered force fold
-//   narrow phase      k_narrow_wave (one wave per pair) and, for the pairs
-//                     too large for a wave, k_narrow (persistent workgroups):
-//                     cull each mesh's triangles against the other mesh's
-//                     box, then a flattened, order-preserving sweep of the
-//                     culled product with the float (outward-rounded) AABB
-//                     test, hits written in (ta, tb) order; k_narrow_exact:
-//                     one thread per hit, the exact FP64 AABB re-test and
-//                     tri-tri; k_narrow_compact: one wave per pair, ballot /
-//                     prefix-sum compaction in the reference's (ta, tb) order
+//                     (one workgroup for up to 256 particles: k_bp_small)
+//   narrow phase      zdx_cluster.h: k_pairs_wave (one wave per pair) and, for
+//                     the pairs too large for a wave, k_pairs_group (a
+//                     workgroup per pair): each mesh's triangle clusters, then
+//                     their triangles, against the other mesh's box, the kept
+//                     ones' float (outward-rounded) boxes in groups;
+//                     k_pairs_exact: one thread per hit, the exact FP64 AABB
+//                     re-test and tri-tri; k_pairs_sort: one wave per pair puts
+//                     its segments in the reference's (ta, tb) order.  Meshes
+//                     beyond 16-bit indices take the kernels of zdx_narrow.h
 //   topology          k_tp_alloc (one thread per pair) and k_tp_pass_a
-//                     (workgroups over flat S^2 test ranges) for the
-//                     quadratic tests; k_tp_snap_cc (one workgroup per pair
-//                     of 40 or more segments: its snap clusters); walks B and
-//                     D with pass C between (components, snap union-find,
-//                     T-junction chains, loops, Sn/Gn/xc0, force) one wave
-//                     per pair with scratch in LDS (zdx_topo.h)
+//                     (zdx_pass_a.h) for the quadratic tests; k_tp_snap_cc
+//                     (one workgroup per pair of 40 or more segments: its snap
+//                     clusters); walks B and D with pass C between (components,
+//                     snap union-find, T-junction chains, loops, Sn/Gn/xc0,
+//                     force) one wave per pair with scratch in LDS (zdx_topo.h)
+//   per-pair call     k_api_begin, then the stages above, k_api_scan and
+//                     k_api_pack: results straight to pinned host memory
 //   k_walls           one wave per particle near a wall: plane sections of
 //                     every candidate wall triangle, clip, area, force
 //   k_fold_integrate  one thread per particle: ordered, atomic-free fold of
@@ -1322,8 +1324,7 @@ struct LaneDev {
 };
 
 // ---- phased topology (zdx_topo.h): pass A, walk B, pass C, walk D.
-// Pass kernels: one 256-thread workgroup per pair of the work list
-// (persistent); walk kernels: one wave per pair, scratch in LDS when it fits,
+// Pass A: persistent workgroups; walk kernels: one wave per pair, scratch in LDS when it fits,
 // else the workgroup's slice of the global scratch.
 
 #include "zdx_pass_a.h"
