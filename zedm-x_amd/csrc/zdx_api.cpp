@@ -1342,21 +1342,23 @@ void contact_pairs_impl(zdx_ctx* c, zdx_ctx::Api& A, const zdx_pair_in* pairs, i
             A.pk_pvtx.ensure((size_t)n + 1); A.pk_tot.ensure(3);
             K.loop_off = A.pk_loop_off.p; K.seg_out_off = A.pk_seg_off.p; K.pvtx_off = A.pk_pvtx.p;
             K.totals = A.pk_tot.p;
-            K.loop_cap = std::max<int64_t>(0, std::min<int64_t>(out->loop_cap, (int64_t)n * T.lmax));
-            K.vtx_cap = want_vtx ? std::max<int64_t>(0, std::min<int64_t>(out->vtx_cap, (int64_t)n * T.vmax)) : 0;
-            K.seg_cap = want_seg ? std::max<int64_t>(0, std::min<int64_t>(out->seg_cap, A.hit_cap)) : 0;
-            K.want_seg = want_seg;
-            auto output = [&](auto& o, auto& buf, int k, int64_t words, bool want) {
+            // rows each array has room for (no more than the buffers can hold)
+            const int64_t loop_cap = std::max<int64_t>(0, std::min<int64_t>(out->loop_cap, (int64_t)n * T.lmax));
+            const int64_t vtx_cap = std::max<int64_t>(0, std::min<int64_t>(out->vtx_cap, (int64_t)n * T.vmax));
+            const int64_t seg_cap = std::max<int64_t>(0, std::min<int64_t>(out->seg_cap, A.hit_cap));
+            auto output = [&](auto& o, auto& buf, int k, int64_t cap, int per, bool want) {
                 using W = std::remove_reference_t<decltype(*o.host)>;
                 if (!want) return;
                 o.host = (W*)slot(c->pin_dev, k);
-                if (words * (int64_t)sizeof(W) > API_SLOT) o.dev = buf.ensure((size_t)words);
+                o.cap = cap;
+                o.per = per;
+                if (o.dev_entries() > 0) o.dev = buf.ensure((size_t)o.dev_entries());
             };
-            output(K.rec_out, A.pk_rec, 6, K.loop_cap * 28, out->loop_rec != nullptr);
-            output(K.ljac_out, A.pk_ljac, 7, K.loop_cap * 72, want_jac);
-            output(K.vtx_out, A.pk_vtx, 8, K.vtx_cap * 3, want_vtx);
-            output(K.vtx_off_out, A.pk_vtx_off, 9, K.loop_cap + 1, want_vtx);
-            output(K.seg_out, A.pk_seg, 10, K.seg_cap * 6, want_seg);
+            output(K.rec_out, A.pk_rec, 6, loop_cap, 28, out->loop_rec != nullptr);
+            output(K.ljac_out, A.pk_ljac, 7, loop_cap, 72, want_jac);
+            output(K.vtx_out, A.pk_vtx, 8, vtx_cap, 3, want_vtx);
+            output(K.vtx_off_out, A.pk_vtx_off, 9, loop_cap + 1, 1, want_vtx);
+            output(K.seg_out, A.pk_seg, 10, seg_cap, 6, want_seg);
             if (columns) {
                 K.h_loop_off = (int32_t*)slot(c->pin_dev, 0); K.h_seg_off = (int32_t*)slot(c->pin_dev, 1);
                 K.h_nseg = (int32_t*)slot(c->pin_dev, 2); K.h_comps = (int32_t*)slot(c->pin_dev, 3);
@@ -1399,19 +1401,19 @@ void contact_pairs_impl(zdx_ctx* c, zdx_ctx::Api& A, const zdx_pair_in* pairs, i
                     copies = true;
                 }
             };
-            auto rows = [&](void* dst, int k, const void* src, int64_t bytes) {
-                fetch(dst, k, bytes <= API_SLOT, src, bytes);
+            auto rows = [&](void* dst, int k, const auto& o, int64_t n_rows) {
+                fetch(dst, k, o.in_slot(n_rows), o.dev, n_rows * o.per * (int64_t)sizeof(*o.host));
             };
             // the large ones are under way while the host copies the others
-            if (out->loop_rec) rows(out->loop_rec, 6, A.pk_rec.p, 8 * 28 * tot[0]);
-            if (want_jac) rows(out->loop_jac, 7, A.pk_ljac.p, 8 * 72 * tot[0]);
+            if (out->loop_rec) rows(out->loop_rec, 6, K.rec_out, tot[0]);
+            if (want_jac) rows(out->loop_jac, 7, K.ljac_out, tot[0]);
             if (want_vtx) {
-                rows(out->vtx_offset, 9, A.pk_vtx_off.p, 4 * (tot[0] + 1));
-                rows(out->loop_vtx, 8, A.pk_vtx.p, 8 * 3 * tot[1]);
+                rows(out->vtx_offset, 9, K.vtx_off_out, tot[0] + 1);
+                rows(out->loop_vtx, 8, K.vtx_out, tot[1]);
             }
             if (want_seg) {
                 fetch(out->seg_offset, 1, columns, A.pk_seg_off.p, 4 * ((int64_t)n + 1));
-                rows(out->segments, 10, A.pk_seg.p, 8 * 6 * tot[2]);
+                rows(out->segments, 10, K.seg_out, tot[2]);
             }
             fetch(out->loop_offset, 0, columns, A.pk_loop_off.p, 4 * ((int64_t)n + 1));
             fetch(out->tri_checks, 5, columns, A.tri_checks.p, 8 * (int64_t)n);

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../../include/zdx.h"
+#include "zdx_api_out.h"
 #include "zdx_internal.h"
 
 namespace zdx {
@@ -276,7 +277,6 @@ void launch_fill_u64(unsigned long long* p, unsigned long long v, int64_t n, hip
 // through its slots, written by the device, so that a call waits for the
 // device once.
 constexpr int64_t API_PIN_IN = (int64_t)1 << 20;
-constexpr int64_t API_SLOT = (int64_t)512 << 10;   // an output array up to this size; a larger one is copied
 constexpr int API_SLOTS = 11;
 constexpr int API_PACK_ONE = 64;                   // calls up to this many pairs are packed by the scanning workgroup
 struct ApiHead {
@@ -286,10 +286,6 @@ struct ApiHead {
 };
 constexpr int64_t API_PIN_BYTES = API_PIN_IN + 4096 + API_SLOTS * API_SLOT;
 static_assert(sizeof(ApiHead) <= 4096, "the header's place");
-template <class T>
-struct ApiOut {
-    T *host = nullptr, *dev = nullptr;
-};
 struct ApiPack {
     int32_t n;                 // pairs
     int32_t lmax, vmax;        // per-pair slots of rec / ljac and of vtx
@@ -309,13 +305,11 @@ struct ApiPack {
     int32_t* seg_out_off;      // n + 1
     int64_t* pvtx_off;         // n + 1: first vertex of each pair's loops
     int64_t* totals;           // loops, vertices, segments
-    ApiOut<double> rec_out;    // loop_cap * 28
-    ApiOut<double> ljac_out;   // loop_cap * 72
-    ApiOut<double> vtx_out;    // vtx_cap * 3
-    ApiOut<int32_t> vtx_off_out;   // loop_cap + 1
-    ApiOut<double> seg_out;    // seg_cap * 6
-    bool want_seg;
-    int64_t loop_cap, vtx_cap, seg_cap;   // rows of the *_out arrays: nothing is written past them
+    ApiOut<double> rec_out;    // 28 a loop
+    ApiOut<double> ljac_out;   // 72 a loop
+    ApiOut<double> vtx_out;    // 3 a vertex
+    ApiOut<int32_t> vtx_off_out;   // one a loop, and the end
+    ApiOut<double> seg_out;    // 6 a segment
     // the per-pair columns' slots (all or none: h_loop_off nullptr)
     int32_t *h_loop_off, *h_seg_off, *h_nseg, *h_comps, *h_raw;
     int64_t* h_checks;

@@ -2044,49 +2044,39 @@ __global__ void __launch_bounds__(256) k_fold_integrate(int32_t n, const double*
     store_body(sout + 16 * (int64_t)i, b);
 }
 
-// The per-pair call's packed output, one pair per wave: each array goes to the
-// caller-visible host memory when it fits its slot there, else to device
-// memory (ApiOut).  A pair whose rows would pass an output's capacity writes
-// nothing to that output (the host then reports the totals and the call fails
-// with ZDX_CAPACITY).
-template <class T>
-__device__ inline T* api_dst(const ApiOut<T>& o, int64_t rows, int per) {
-    return o.host && rows * per * (int64_t)sizeof(T) <= API_SLOT ? o.host : o.dev;
-}
+// The per-pair call's packed output, one pair per wave: each array goes where
+// ApiOut says, and an array with more rows than its capacity nowhere (the host
+// then reports the totals and the call fails with ZDX_CAPACITY).
 __device__ inline void api_pack_pair(const ApiPack& k, int64_t p, int lane) {
     const int64_t L = k.totals[0];
     const int nl = k.nloops[p];
     const int64_t lo = k.loop_off[p];
-    double* rec = api_dst(k.rec_out, L, 28);
-    double* ljac = api_dst(k.ljac_out, L, 72);
-    if (lo + nl <= k.loop_cap) {
-        if (rec)
-            for (int64_t e = lane; e < 28 * (int64_t)nl; e += WAVE) rec[28 * lo + e] = k.rec[(p * k.lmax) * 28 + e];
-        if (ljac)
-            for (int64_t e = lane; e < 72 * (int64_t)nl; e += WAVE) ljac[72 * lo + e] = k.ljac[(p * k.lmax) * 72 + e];
-    }
-    if (k.vtx) {
-        double* vtx = api_dst(k.vtx_out, k.totals[1], 3);
-        int32_t* off = api_dst(k.vtx_off_out, L + 1, 1);
-        const int64_t vo = k.pvtx_off[p];
-        const int64_t nv = k.pvtx_off[p + 1] - vo;
-        if (lane == 0 && lo + nl <= k.loop_cap) {
-            int64_t acc = vo;
-            for (int l = 0; l < nl; ++l) {
-                off[lo + l] = (int32_t)acc;
-                acc += (int64_t)k.rec[(p * k.lmax + l) * 28 + 24];
-            }
-            if (p == k.n - 1) off[lo + nl] = (int32_t)acc;
+    double* rec = k.rec_out.at(L);
+    double* ljac = k.ljac_out.at(L);
+    if (rec)
+        for (int64_t e = lane; e < 28 * (int64_t)nl; e += WAVE) rec[28 * lo + e] = k.rec[(p * k.lmax) * 28 + e];
+    if (ljac)
+        for (int64_t e = lane; e < 72 * (int64_t)nl; e += WAVE) ljac[72 * lo + e] = k.ljac[(p * k.lmax) * 72 + e];
+    const int64_t vo = k.pvtx_off[p];
+    int32_t* off = k.vtx_off_out.at(L + 1);
+    if (off && lane == 0) {
+        int64_t acc = vo;
+        for (int l = 0; l < nl; ++l) {
+            off[lo + l] = (int32_t)acc;
+            acc += (int64_t)k.rec[(p * k.lmax + l) * 28 + 24];
         }
-        if (vo + nv <= k.vtx_cap)
-            for (int64_t e = lane; e < 3 * nv; e += WAVE) vtx[3 * vo + e] = k.vtx[(p * k.vmax) * 3 + e];
+        if (p == k.n - 1) off[lo + nl] = (int32_t)acc;
     }
-    if (k.want_seg) {
-        double* seg = api_dst(k.seg_out, k.totals[2], 6);
+    double* vtx = k.vtx_out.at(k.totals[1]);
+    if (vtx) {
+        const int64_t nv = k.pvtx_off[p + 1] - vo;
+        for (int64_t e = lane; e < 3 * nv; e += WAVE) vtx[3 * vo + e] = k.vtx[(p * k.vmax) * 3 + e];
+    }
+    double* seg = k.seg_out.at(k.totals[2]);
+    if (seg) {
         const int64_t so = k.seg_out_off[p];
         const int ns = k.nseg[p];
-        if (so + ns <= k.seg_cap)
-            for (int64_t e = lane; e < 6 * (int64_t)ns; e += WAVE) seg[6 * so + e] = k.arena[6 * k.seg_off[p] + e];
+        for (int64_t e = lane; e < 6 * (int64_t)ns; e += WAVE) seg[6 * so + e] = k.arena[6 * k.seg_off[p] + e];
     }
     // the per-pair columns
     if (k.h_loop_off) {
