@@ -61,8 +61,8 @@ __device__ inline void pass_a_unit(const double* seg, const int* c9, const float
     const int tid = threadIdx.x, lane = lane_id(), wid = uni(tid / WAVE);
     const uint64_t below = (1ull << lane) - 1ull;
     int* rows = cntp + S;
-    const int npt = S * (2 * S - 1);   // endpoint pairs of 2S points
-    const int nw = (npt + 63) >> 6;
+    const int64_t npt = (int64_t)S * (2 * S - 1);   // endpoint pairs of 2S points: past 31 bits at 32769 segments
+    const int nw = (int)((npt + 63) >> 6);
     auto meet = [&](int i, int j) {
         bool r = true;
         if (STAGED) {
@@ -82,7 +82,7 @@ __device__ inline void pass_a_unit(const double* seg, const int* c9, const float
     // rows [ra, rb) by the workgroup's waves: their adjacency (adj), or only
     // j <= i; and the snap hits in words [c0, c1)
     auto sweep = [&](int ra, int rb, bool adj, int c0, int c1) {
-        const int tb = 64 * c0, te = 64 * c1 < npt ? 64 * c1 : npt;
+        const int64_t tb = 64 * (int64_t)c0, te = 64 * (int64_t)c1 < npt ? 64 * (int64_t)c1 : npt;
         const int r0 = ra + (int)((int64_t)(rb - ra) * wid / NW), r1 = ra + (int)((int64_t)(rb - ra) * (wid + 1) / NW);
         int crow = -1, ccnt = 0;   // the row that the last tested pair belonged to, and its count so far
         auto test = [&](int n) {   // the first n <= WAVE pairs of the list
@@ -111,7 +111,8 @@ __device__ inline void pass_a_unit(const double* seg, const int* c9, const float
             if (on && e.y <= e.x && c1 > c0) {
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    const int a = 2 * e.x + (q >> 1), c = 2 * e.y + (q & 1), t = a * (a - 1) / 2 + c;
+                    const int a = 2 * e.x + (q >> 1), c = 2 * e.y + (q & 1);
+                    const int64_t t = (int64_t)a * (a - 1) / 2 + c;   // a (a - 1): past 31 bits at 23171 segments
                     if (c < a && t >= tb && t < te && tp_snap_hit(seg, c9, h, a, c))
                         atomicOr(&sw[(t >> 6) - c0], 1ull << (t & 63));
                 }
