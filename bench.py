@@ -12,13 +12,13 @@ integrator).  300 untimed steps settle the bed first, whatever --warmup
 says (the lattice-seeded bed reaches its colliding state of about 12k
 candidate pairs per step within that), the autotuner picks the narrow-phase
 shape on the settled state, W more untimed warmup steps follow, then K timed
-steps in batched mode (persistent work queue, hipGraph-captured step), then
+steps in batched mode (persistent work queue, no host read within a step), then
 the same K steps again in plain mode (one kernel per stage, host-sized
 launches) from a checkpoint of the post-warmup state; the two trajectories
 must be bitwise equal.  value = contact pairs/s of the batched step, where a
 contact pair is a broad-phase candidate pair evaluated by the narrow phase.
 The line also carries steps/s, the per-step counters, the steps run again
-after a buffer growth and the graph captures inside the timed window, the
+after a buffer growth inside the timed window, the
 narrow phase's roofline and the single-thread reference CPU baseline.
 
 Prints one JSON line.  --gpus N with N > 1 exits: the step runs on one GPU.
@@ -239,7 +239,7 @@ def uneven_block(ctx, reps: int, cpu_sample: int, log):
 def packing_block(ctx, steps: int, log):
     """The 1M-particle concave packing (zdx.workloads.concave_packing: 16
     star templates of 320-2560 triangles, radii 1-4 mm, 0.5 m box, dt 5e-6)
-    on the same GPU: 2 untimed batched steps (buffer growth, graph capture),
+    on the same GPU: 2 untimed batched steps (buffer growth),
     then `steps` timed batched steps."""
     import zdx
     from zdx import workloads as W
@@ -356,7 +356,7 @@ def summarize_profiles(stats_dir, fetch_dir, write_dir, command="", timed_stats=
     for f in glob.glob(os.path.join(stats_dir, "*kernel_stats.csv")):
         stats += list(csv.DictReader(open(f)))
     stats.sort(key=lambda r: -float(r["TotalDurationNs"]))
-    lines = ["# Kernel durations -- granular bed, 100k polyhedra, batched step (graph capture off)", "",
+    lines = ["# Kernel durations -- granular bed, 100k polyhedra, batched step", "",
              f"Command: `{command}`" if command else "", "",
              "| kernel | calls | average us | total % |", "|---|---|---|---|"]
     for r in stats[:30]:
@@ -471,7 +471,7 @@ def summarize_valu(pmc_dir, stats_dir, command="", timed=5, n_cu=256):
                          fp64=m["SQ_INSTS_VALU_FLOPS_FP64"],
                          fp64_tflops=m["SQ_INSTS_VALU_FLOPS_FP64"] / (t_us * 1e-6) / 1e12 if t_us > 0 else 0.0))
     rows.sort(key=lambda r: -r["t_us"])
-    lines = ["# VALU and occupancy -- granular bed, 100k polyhedra, batched step (graph capture off)", "",
+    lines = ["# VALU and occupancy -- granular bed, 100k polyhedra, batched step", "",
              f"Command: `{command}`" if command else "", "",
              f"Counters: {' '.join(VALU_COUNTERS)} (one --pmc pass), per kernel averaged over its last {timed} "
              f"dispatches (the timed steps); durations from the kernel trace of the same bench.  VALUBusy, "
@@ -564,16 +564,14 @@ def main():
     log(f"setup {time.time() - t0:.1f}s: {wl.n} particles, {n_meshes} meshes")
 
     # settle (untimed, fixed length), then the autotune on the settled
-    # state, then the warmup (the first step after the autotune captures the
-    # graphs again)
+    # state, then the warmup
     tiles = None
     if args.tiles:
         tiles = [int(x) for x in args.tiles.split(",")]
         sim.set_tiles(tiles[0], tiles[1])
     sim.step(args.settle, zdx.MODE_BATCHED)
     st_settle = sim.stage_times()
-    log(f"settle {args.settle} steps done {time.time() - t0:.1f}s, retries {st_settle['retries']}, "
-        f"graph captures {st_settle['graph_captures']}")
+    log(f"settle {args.settle} steps done {time.time() - t0:.1f}s, retries {st_settle['retries']}")
     if not args.tiles and not args.no_autotune:
         tiles = list(sim.autotune())
         log(f"autotune: threads*100+tests={tiles[0]} groups/CU={tiles[1]}")
@@ -672,7 +670,7 @@ def main():
                                f"12-triangle box wall, gravity -9.81, dt 1e-5, agitated non-overlapping seeding; "
                                f"timed after {args.settle} untimed settle steps, the autotune on the settled "
                                f"state and {warm} warmup steps",
-                   "particles": wl.n, "meshes": n_meshes, "mode": "batched (persistent queue + hipGraph)",
+                   "particles": wl.n, "meshes": n_meshes, "mode": "batched (persistent queue)",
                    "tiles": tiles, "settle_steps": args.settle},
         "steps_per_s": args.steps / tb,
         "contact_pairs_per_step": pairs_b / args.steps,

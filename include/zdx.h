@@ -208,9 +208,9 @@ enum {
     ZDX_N_COUNTERS = 12
 };
 /* Runs n_steps steps in mode ZDX_MODE_PLAIN (one kernel per stage,
- * host-sized launches) or ZDX_MODE_BATCHED (persistent work-queue kernels,
- * whole step captured in a hipGraph).  counters (may be NULL) receives the
- * counters of the last step. */
+ * host-sized launches) or ZDX_MODE_BATCHED (persistent work-queue kernels, no
+ * host read within a step).  counters (may be NULL) receives the counters of
+ * the last step. */
 zdx_status zdx_sim_step(zdx_sim* sim, int32_t n_steps, int32_t mode, int64_t* counters);
 
 /* Per particle 16 doubles: pos(3) quat(4) vel(3) omega(3) L(3). */
@@ -243,14 +243,14 @@ zdx_status zdx_sim_restore(zdx_sim* sim, const char* path);
 /* Stage timing and counters accumulated over the steps since the previous
  * call, then reset.  Each stage's kernels stamp their span (earliest
  * workgroup start, latest wave end) on the device's constant-rate clock, in
- * both modes and inside the captured graph.  out[0..5]:
+ * both modes.  out[0..5]:
  * mean ms per step of transform, broad phase, narrow phase, topology+forces,
  * walls, fold+integrate+counters; out[6]: steps; out[7..7+ZDX_N_COUNTERS):
  * counter sums (ZDX_CTR_SEG_MAX: the maximum); out[7+ZDX_N_COUNTERS]: mean ms
  * of the narrow-phase kernels alone (without the work ordering);
  * out[8+ZDX_N_COUNTERS]: steps run again after a buffer growth;
- * out[9+ZDX_N_COUNTERS]: captures of the batched step's graphs (a growth or a
- * parameter change invalidates them).  The walls run on a second stream
+ * out[9+ZDX_N_COUNTERS]: 0 (steps are launched directly, no graphs are
+ * captured).  The walls run on a second stream
  * alongside the narrow phase and the topology, so the stages can add up to
  * more than the step.  Writes min(n, 10 + ZDX_N_COUNTERS) values. */
 zdx_status zdx_sim_stage_times(zdx_sim* sim, double* out, int32_t n);

@@ -51,7 +51,7 @@ constexpr int WAVE = 64;
 
 // Stage stamps: one thread writes the device's constant-rate clock into a
 // slot; launched on the stream between stages, so consecutive stamps bracket
-// a stage (kernels of a stream run in order, also inside a captured graph).
+// a stage (kernels of a stream run in order).
 // A per-kernel scheme with an atomic from every wave would serialise tens of
 // thousands of same-address atomics per launch.
 __global__ void k_stamp(unsigned long long* slot) { *slot = (unsigned long long)wall_clock64(); }
