@@ -94,6 +94,17 @@ struct DBuf {
 struct MeshRec {
     HostMesh h;
     double tol, area_eps;
+    int32_t shape = -1;   // index in zdx_ctx::shapes, from the first upload on
+};
+
+// What meshes with the same triangle indices (scaled copies of one shape)
+// share: their triangles and clusters, in the device's numbering of the
+// vertices.  Made once, at the upload after the first such mesh.
+struct MeshShape {
+    int32_t mesh;                // the first of them
+    std::vector<int32_t> from;   // device vertex -> host vertex
+    std::vector<int32_t> tri;    // device vertices, 3 per triangle
+    std::vector<Cluster> clusters;
 };
 
 // Device buffers of the phased topology (zdx_topo.h), used by the time step
@@ -206,15 +217,11 @@ struct zdx_ctx {
     bool mesh_dirty = true;
     uint64_t mesh_version = 0;
     int32_t max_tris = 1;
-    // device mesh store
-    DBuf<double> m_verts;
-    DBuf<int32_t> m_tri;
-    DBuf<int32_t> m_voff, m_nv, m_toff, m_nt;
-    DBuf<double> m_tol, m_aeps;
-    DBuf<int32_t> m_soff, m_ns, m_susp;
-    DBuf<Cluster> m_clus;
-    DBuf<float> m_sph;
-    DBuf<int32_t> m_nc, m_coff, m_sphoff;
+    std::vector<MeshShape> shapes;
+    std::unordered_map<uint64_t, std::vector<int32_t>> shapes_of;   // hash of the triangle indices -> shapes
+    // device mesh store: one block and the views into it
+    DBuf<char> m_store;
+    DMeshes m_view{};
     bool clusters = false;   // every mesh on the device has its clusters (else the hit-arena kernels run)
     // per-pair API buffers (api: grown with hipMalloc; api_na: carved from
     // na_arena, this device's no-allocation scratch, at every call)
@@ -283,101 +290,118 @@ struct zdx_ctx {
     void* scratch_dev = nullptr;   // this device's `scratch` array
     Arena na_arena;
 
-    DMeshes dmeshes() {
-        DMeshes M;
-        M.verts = m_verts.p; M.tri_idx = m_tri.p; M.vert_off = m_voff.p; M.nverts = m_nv.p;
-        M.tri_off = m_toff.p; M.ntris = m_nt.p; M.tol = m_tol.p; M.area_eps = m_aeps.p;
-        M.susp_off = m_soff.p; M.nsusp = m_ns.p; M.susp = m_susp.p;
-        M.clusters = clusters ? m_clus.p : nullptr;
-        M.clus_sph = m_sph.p; M.nclus = m_nc.p; M.clus_off = m_coff.p; M.sph_off = m_sphoff.p;
-        return M;
+    const DMeshes& dmeshes() const { return m_view; }
+    // The shape of meshes[k], made if it is the first mesh of its shape.  The
+    // vertices are numbered in the clusters' order, so that a cluster's lie
+    // together.
+    int32_t shape_of(int32_t k) {
+        MeshRec& m = meshes[k];
+        if (m.shape >= 0) return m.shape;
+        uint64_t hsh = 1469598103934665603ull ^ m.h.tri_idx.size();
+        for (int32_t x : m.h.tri_idx) hsh = (hsh ^ (uint32_t)x) * 1099511628211ull;
+        std::vector<int32_t>& same = shapes_of[hsh];
+        for (int32_t o : same)
+            if (meshes[shapes[o].mesh].h.tri_idx == m.h.tri_idx) return m.shape = o;
+        MeshShape s;
+        s.mesh = k;
+        if (clusters) s.clusters = cluster_mesh(m.h);
+        std::vector<int32_t> to(m.h.verts.size() / 3, -1);
+        auto number = [&](int32_t x) {
+            if (to[x] < 0) {
+                to[x] = (int32_t)s.from.size();
+                s.from.push_back(x);
+            }
+            return to[x];
+        };
+        for (Cluster& q : s.clusters)
+            for (uint16_t& x : q.v) x = (uint16_t)number(x);
+        s.tri.reserve(m.h.tri_idx.size());
+        for (int32_t x : m.h.tri_idx) s.tri.push_back(number(x));
+        same.reserve(same.size() + 1);
+        shapes.push_back(std::move(s));
+        same.push_back((int32_t)shapes.size() - 1);
+        return m.shape = (int32_t)shapes.size() - 1;
     }
     void sync_meshes() {
         if (!mesh_dirty) return;
-        std::vector<double> v;
-        std::vector<int32_t> t, voff, nv, toff, nt;
-        std::vector<double> tol, aeps;
-        std::vector<int32_t> soff, ns, susp;
-        // meshes with the same triangle indices (scaled copies of one shape)
-        // share one copy on the device, so that the narrow phase's index
-        // loads stay in cache.  So do a shape's clusters, and its vertices are
-        // numbered in their order on the device, so that a cluster's vertices
-        // lie together
-        struct Shape {
-            const std::vector<int32_t>* idx;
-            int32_t at, cl, ncl;         // its first triangle, its clusters
-            std::vector<int32_t> from;   // device vertex -> host vertex
-        };
-        std::unordered_map<uint64_t, std::vector<int32_t>> seen;   // hash -> shapes
-        std::vector<Shape> shapes;
-        std::vector<Cluster> cl;
-        std::vector<int32_t> nc, coff, sphoff;
-        int32_t nsph = 0;
+        const size_t nm = meshes.size();
         clusters = true;
         for (auto& m : meshes)
             clusters = clusters && m.h.tri_idx.size() / 3 <= CLUSTER_MAX_TRIS &&
                        m.h.verts.size() / 3 <= CLUSTER_MAX_VERTS;
-        for (auto& m : meshes) {
-            soff.push_back((int32_t)susp.size());
-            ns.push_back((int32_t)m.h.suspect.size());
-            susp.insert(susp.end(), m.h.suspect.begin(), m.h.suspect.end());
-            voff.push_back((int32_t)(v.size() / 3));
-            nv.push_back((int32_t)(m.h.verts.size() / 3));
-            nt.push_back((int32_t)(m.h.tri_idx.size() / 3));
-            uint64_t hsh = 1469598103934665603ull ^ m.h.tri_idx.size();
-            for (int32_t x : m.h.tri_idx) hsh = (hsh ^ (uint32_t)x) * 1099511628211ull;
-            int32_t sh = -1;
-            for (int32_t o : seen[hsh])
-                if (*shapes[o].idx == m.h.tri_idx) { sh = o; break; }
-            if (sh < 0) {
-                sh = (int32_t)shapes.size();
-                seen[hsh].push_back(sh);
-                std::vector<Cluster> q;
-                if (clusters) q = cluster_mesh(m.h);
-                Shape s{&m.h.tri_idx, (int32_t)(t.size() / 3), (int32_t)cl.size(), (int32_t)q.size(), {}};
-                std::vector<int32_t> to(m.h.verts.size() / 3, -1);
-                auto number = [&](int32_t x) {
-                    if (to[x] < 0) {
-                        to[x] = (int32_t)s.from.size();
-                        s.from.push_back(x);
-                    }
-                    return to[x];
-                };
-                for (Cluster& k : q)
-                    for (uint16_t& x : k.v) x = (uint16_t)number(x);
-                for (int32_t x : m.h.tri_idx) t.push_back(number(x));
-                cl.insert(cl.end(), q.begin(), q.end());
-                shapes.push_back(std::move(s));
-            }
-            for (int32_t x : shapes[sh].from)
-                v.insert(v.end(), m.h.verts.begin() + 3 * (size_t)x, m.h.verts.begin() + 3 * (size_t)x + 3);
-            nc.push_back(shapes[sh].ncl);
-            coff.push_back(shapes[sh].cl);
-            sphoff.push_back(nsph);
-            nsph += shapes[sh].ncl;
-            toff.push_back(shapes[sh].at);
-            tol.push_back(m.tol);
-            aeps.push_back(m.area_eps);
+        size_t nv = 0, ns = 0, nt = 0, nc = 0, nsph = 0;
+        for (size_t k = 0; k < nm; ++k) {
+            const MeshShape& sh = shapes[shape_of((int32_t)k)];
+            nv += sh.from.size();
+            ns += meshes[k].h.suspect.size();
+            nsph += sh.clusters.size();
         }
-        m_verts.upload(v.data(), v.size(), stream);
-        m_tri.upload(t.data(), t.size(), stream);
-        m_voff.upload(voff.data(), voff.size(), stream);
-        m_nv.upload(nv.data(), nv.size(), stream);
-        m_toff.upload(toff.data(), toff.size(), stream);
-        m_nt.upload(nt.data(), nt.size(), stream);
-        m_tol.upload(tol.data(), tol.size(), stream);
-        m_aeps.upload(aeps.data(), aeps.size(), stream);
-        m_soff.upload(soff.data(), soff.size(), stream);
-        m_ns.upload(ns.data(), ns.size(), stream);
-        m_susp.upload(susp.data(), susp.size(), stream);
-        if (clusters) {
-            m_clus.upload(cl.data(), cl.size(), stream);
-            m_nc.upload(nc.data(), nc.size(), stream);
-            m_coff.upload(coff.data(), coff.size(), stream);
-            m_sphoff.upload(sphoff.data(), sphoff.size(), stream);
-            m_sph.ensure(4 * (size_t)nsph);
-            launch_cluster_spheres(dmeshes(), (int32_t)meshes.size(), m_sph.p, stream);
+        for (auto& sh : shapes) {
+            nt += sh.tri.size();
+            nc += sh.clusters.size();
         }
+        // the store's parts, then the whole in one copy (the spheres are made on
+        // the device)
+        size_t bytes = 0;
+        auto part = [&](size_t n, size_t each) {
+            const size_t at = bytes;
+            bytes = (bytes + n * each + 255) & ~(size_t)255;
+            return at;
+        };
+        const size_t o_v = part(3 * nv, 8), o_tol = part(nm, 8), o_aeps = part(nm, 8), o_t = part(nt, 4),
+                     o_s = part(ns, 4), o_voff = part(nm, 4), o_nv = part(nm, 4), o_toff = part(nm, 4),
+                     o_nt = part(nm, 4), o_soff = part(nm, 4), o_ns = part(nm, 4), o_nc = part(nm, 4),
+                     o_coff = part(nm, 4), o_sph0 = part(nm, 4), o_c = part(nc, sizeof(Cluster)), up = bytes,
+                     o_sph = part(4 * nsph, 4);
+        std::vector<char> host(up);
+        auto ints = [&](size_t o) { return (int32_t*)(host.data() + o); };
+        std::vector<int32_t> tri0(shapes.size()), clus0(shapes.size());
+        size_t at_t = 0, at_c = 0;
+        for (size_t k = 0; k < shapes.size(); ++k) {
+            const MeshShape& sh = shapes[k];
+            tri0[k] = (int32_t)(at_t / 3);
+            clus0[k] = (int32_t)at_c;
+            std::copy(sh.tri.begin(), sh.tri.end(), ints(o_t) + at_t);
+            std::copy(sh.clusters.begin(), sh.clusters.end(), (Cluster*)(host.data() + o_c) + at_c);
+            at_t += sh.tri.size();
+            at_c += sh.clusters.size();
+        }
+        double* v = (double*)(host.data() + o_v);
+        size_t at_v = 0, at_s = 0, at_sph = 0;
+        for (size_t k = 0; k < nm; ++k) {
+            const MeshRec& m = meshes[k];
+            const MeshShape& sh = shapes[m.shape];
+            ints(o_voff)[k] = (int32_t)at_v;
+            ints(o_nv)[k] = (int32_t)sh.from.size();
+            ints(o_toff)[k] = tri0[m.shape];
+            ints(o_nt)[k] = (int32_t)(sh.tri.size() / 3);
+            ints(o_soff)[k] = (int32_t)at_s;
+            ints(o_ns)[k] = (int32_t)m.h.suspect.size();
+            ints(o_nc)[k] = (int32_t)sh.clusters.size();
+            ints(o_coff)[k] = clus0[m.shape];
+            ints(o_sph0)[k] = (int32_t)at_sph;
+            ((double*)(host.data() + o_tol))[k] = m.tol;
+            ((double*)(host.data() + o_aeps))[k] = m.area_eps;
+            for (size_t x = 0; x < sh.from.size(); ++x)
+                std::memcpy(v + 3 * (at_v + x), m.h.verts.data() + 3 * (size_t)sh.from[x], 24);
+            std::copy(m.h.suspect.begin(), m.h.suspect.end(), ints(o_s) + at_s);
+            at_v += sh.from.size();
+            at_s += m.h.suspect.size();
+            at_sph += sh.clusters.size();
+        }
+        m_store.ensure(bytes);
+        if (up) HIPC(hipMemcpyAsync(m_store.p, host.data(), up, hipMemcpyHostToDevice, stream));
+        auto dev = [&](size_t o) { return (int32_t*)(m_store.p + o); };
+        DMeshes M{};
+        M.verts = (const double*)(m_store.p + o_v); M.tri_idx = dev(o_t); M.vert_off = dev(o_voff); M.nverts = dev(o_nv);
+        M.tri_off = dev(o_toff); M.ntris = dev(o_nt);
+        M.tol = (const double*)(m_store.p + o_tol); M.area_eps = (const double*)(m_store.p + o_aeps);
+        M.susp_off = dev(o_soff); M.nsusp = dev(o_ns); M.susp = dev(o_s);
+        M.clusters = clusters ? (const Cluster*)(m_store.p + o_c) : nullptr;
+        M.clus_sph = (const float*)(m_store.p + o_sph); M.nclus = dev(o_nc); M.clus_off = dev(o_coff);
+        M.sph_off = dev(o_sph0);
+        m_view = M;
+        if (clusters) launch_cluster_spheres(M, (int32_t)nm, (float*)(m_store.p + o_sph), stream);
         HIPC(hipStreamSynchronize(stream));
         mesh_dirty = false;
         ++mesh_version;
