@@ -127,8 +127,21 @@ struct TopoWork {
     int64_t slices = 0;
     int32_t slice_seg_max = 0;
 
+    // The buffers that the narrow phase's cluster path borrows, being done with
+    // them when the topology starts: its hits (32 bytes a slot) lie where pass A
+    // puts the cells (36), its segments before they are in order (48) where
+    // walk B puts the vertices (48).
+    void ensure_narrow(int64_t segs) { cell9.ensure(9 * (size_t)segs); V.ensure(6 * (size_t)segs); }
+    int32_t* hits() const { return cell9.p; }
+    double* seg_tmp() const { return V.p; }
+    static_assert(sizeof(PairHit) <= 9 * sizeof(int32_t), "a hit fits its segment's cells");
+    bool arena_holds(int64_t segs) const {
+        return comp.n >= TPC_N * (size_t)segs && vcell.n >= 6 * (size_t)segs && E.n >= 2 * (size_t)segs &&
+               lab.n >= 2 * (size_t)segs;
+    }
     void ensure_arena(int64_t segs) {
-        cell9.ensure(9 * (size_t)segs); comp.ensure(TPC_N * (size_t)segs); V.ensure(6 * (size_t)segs);
+        ensure_narrow(segs);
+        comp.ensure(TPC_N * (size_t)segs);
         vcell.ensure(6 * (size_t)segs); E.ensure(2 * (size_t)segs); lab.ensure(2 * (size_t)segs);
     }
     void ensure_items(int64_t items) {
@@ -234,8 +247,6 @@ struct zdx_ctx {
         DBuf<int32_t> nondeg;
         DBuf<int32_t> pi, pj, order, npairs, status;
         DBuf<NarrowItem> items;
-        DBuf<PairItem> pitems;
-        DBuf<double> seg_tmp;
         DBuf<unsigned long long> stamps;
         DBuf<int64_t> seg_off, tri_checks, tri_tests;
         DBuf<int32_t> nseg, tri_hits, tri_scanned;
@@ -265,7 +276,7 @@ struct zdx_ctx {
         template <class F>
         void each_buf(F&& f) {
             f(pairs_in); f(mesh); f(state); f(wv_off); f(wt_off); f(wv); f(aabb); f(nondeg); f(pi); f(pj); f(order);
-            f(npairs); f(status); f(items); f(pitems); f(seg_tmp); f(stamps); f(seg_off); f(tri_checks); f(tri_tests); f(nseg); f(tri_hits);
+            f(npairs); f(status); f(items); f(stamps); f(seg_off); f(tri_checks); f(tri_tests); f(nseg); f(tri_hits);
             f(tri_scanned); f(arena); f(list_i); f(list_f); f(hits); f(hit_tri); f(hit_flag); f(hit_top); f(hit_off);
             f(queue); f(heavy); f(bcnt); f(bcur); f(ncontrib); f(comps); f(loops_raw); f(tstatus); f(topo_list); f(topo_n);
             f(status2); f(rec); f(vtx); f(prov); f(ej); f(vj); f(ljac); f(pk_loop_off); f(pk_seg_off);
@@ -537,7 +548,6 @@ struct zdx_sim {
     DBuf<int32_t> d_order, d_bcnt, d_bcur, d_topo_list, d_topo_n, d_topo_big, d_topo_small, d_topo_nbs;
     DBuf<NarrowItem> d_items;
     DBuf<PairItem> d_pitems;
-    DBuf<double> d_seg_tmp;
     DBuf<int64_t> d_seg_off, d_tri_checks, d_tri_tests;
     DBuf<int32_t> d_nseg, d_tri_hits, d_tri_scanned;
     DBuf<double> d_arena;        // segments, one slot per hit slot
@@ -626,13 +636,13 @@ struct zdx_sim {
         P.cap = pair_cap; P.n = ps[par].n.p; P.pi = ps[par].pi.p; P.pj = ps[par].pj.p;
         P.order = lpt ? d_order.p : nullptr;
         P.items = lpt ? d_items.p : nullptr;
-        P.pitems = d_pitems.p; P.seg_tmp = d_seg_tmp.p;
+        if (ctx->clusters) { P.pitems = d_pitems.p; P.seg_tmp = tw.seg_tmp(); }
         P.seg_off = d_seg_off.p; P.nseg = d_nseg.p; P.tri_checks = d_tri_checks.p; P.tri_tests = d_tri_tests.p;
         P.tri_hits = d_tri_hits.p; P.tri_scanned = d_tri_scanned.p; P.arena = d_arena.p; P.arena_cap = hit_cap;
         P.status = d_status.p;
         P.topo_list = d_topo_list.p; P.topo_n = d_topo_n.p;
         P.topo_big = d_topo_big.p; P.topo_small = d_topo_small.p; P.n_big = d_topo_nbs.p; P.n_small = d_topo_nbs.p + 1;
-        P.hits = d_hits.p; P.hit_cap = hit_cap; P.hit_top = d_hit_top.p; P.hit_off = d_hit_off.p;
+        P.hits = ctx->clusters ? tw.hits() : d_hits.p; P.hit_cap = hit_cap; P.hit_top = d_hit_top.p; P.hit_off = d_hit_off.p;
         P.hit_shards = (int32_t)std::min<int64_t>(HIT_SHARDS, hit_cap);
         P.hit_flag = d_hit_flag.p;
         P.heavy = d_heavy.p;
@@ -693,7 +703,7 @@ struct zdx_sim {
             HIPC(hipMemcpy(ps[k].n.p, &n, sizeof(int32_t), hipMemcpyHostToDevice));
         }
         d_adj_j.ensure(adj_cap); d_adj_pair.ensure(adj_cap);
-        d_order.ensure(cap); d_items.ensure(cap); d_pitems.ensure(cap); d_heavy.ensure(cap); d_topo_list.ensure(cap); d_topo_n.ensure(1);
+        d_order.ensure(cap); d_heavy.ensure(cap); d_topo_list.ensure(cap); d_topo_n.ensure(1);
         d_topo_big.ensure(cap); d_topo_small.ensure(cap); d_topo_nbs.ensure(2);
         d_hit_off.ensure(cap); d_hit_top.ensure(HIT_SHARDS * HIT_TOP_STRIDE);
         d_seg_off.ensure(cap); d_tri_checks.ensure(cap); d_tri_tests.ensure(cap);
@@ -701,6 +711,7 @@ struct zdx_sim {
         d_ncontrib.ensure(cap); d_comps.ensure(cap); d_loops_raw.ensure(cap); d_tstatus.ensure(cap);
         d_contrib.ensure((size_t)cap * lmax * 9);
         tw.ensure_items(cap);
+        ensure_narrow();
     }
     void alloc_lmax(int32_t l) {
         lmax = l;
@@ -714,21 +725,22 @@ struct zdx_sim {
     }
     void alloc_hits(int64_t cap) {
         hit_cap = cap;
-        d_hits.release(); d_hit_flag.release(); d_arena.release(); d_seg_tmp.release();
+        d_hits.release(); d_hit_flag.release(); d_arena.release();
         d_arena.ensure(6 * (size_t)cap);
         tw.ensure_arena(cap);
-        ensure_hits();
+        ensure_narrow();
     }
-    // the narrow phase's hits: 32 bytes each and their segments' place on the
-    // cluster path, 24 bytes on the hit-arena path, which also needs its
-    // workgroups' lists of kept triangles
-    void ensure_hits() {
-        d_hits.ensure((ctx->clusters ? 8 : 6) * (size_t)hit_cap);
+    // what the narrow phase needs of its own: the work items of its path and,
+    // on the hit-arena path, the hits (on the cluster path they lie in the
+    // topology's buffers) and the workgroups' lists of kept triangles
+    void ensure_narrow() {
         d_hit_flag.ensure((size_t)hit_cap);
         if (ctx->clusters) {
-            d_seg_tmp.ensure(6 * (size_t)hit_cap);
+            d_pitems.ensure(pair_cap);
             return;
         }
+        d_items.ensure(pair_cap);
+        d_hits.ensure(6 * (size_t)hit_cap);
         const size_t groups = (size_t)std::max(1, ctx->n_cu * 16);
         d_list_i.ensure(groups * 8 * (size_t)tmax);
         d_list_f.ensure(groups * 12 * (size_t)tmax);
@@ -1090,7 +1102,7 @@ void step_once(zdx_sim* s, bool batched) {
     s->ctx->sync_meshes();
     if (s->mesh_version != s->ctx->mesh_version) {
         s->mesh_version = s->ctx->mesh_version;
-        s->ensure_hits();
+        s->ensure_narrow();
     }
     for (int attempt = 0; attempt < 12; ++attempt) {
         const int par = s->parity;
@@ -1204,8 +1216,7 @@ void contact_pairs_impl(zdx_ctx* c, zdx_ctx::Api& A, const zdx_pair_in* pairs, i
         DBodies B;
         B.n = nb; B.mesh = A.mesh.p; B.state = A.state.p; B.wv_off = A.wv_off.p; B.wt_off = A.wt_off.p;
         B.wv = A.wv.p; B.nondeg = A.nondeg.p; B.aabb = A.aabb.p;
-        A.pi.ensure(n); A.pj.ensure(n); A.npairs.ensure(1); A.status.ensure(1); A.order.ensure(n); A.items.ensure(n);
-        A.pitems.ensure(n); A.stamps.ensure(4);
+        A.pi.ensure(n); A.pj.ensure(n); A.npairs.ensure(1); A.status.ensure(1); A.order.ensure(n); A.stamps.ensure(4);
         A.status2.ensure(1);
         A.seg_off.ensure(n); A.tri_checks.ensure(n); A.tri_tests.ensure(n); A.nseg.ensure(n); A.tri_hits.ensure(n); A.tri_scanned.ensure(n);
         A.queue.ensure(NARROW_COUNTERS); A.heavy.ensure(n); A.bcnt.ensure(64); A.bcur.ensure(64);
@@ -1216,6 +1227,7 @@ void contact_pairs_impl(zdx_ctx* c, zdx_ctx::Api& A, const zdx_pair_in* pairs, i
         int groups = std::min<int>(persistent_groups(c, 8), std::max(1, n));
         groups = (int)std::max<int64_t>(1, std::min<int64_t>(groups, lim.list_bytes / (80 * (int64_t)c->max_tris)));
         if (!c->clusters) {
+            A.items.ensure(n);
             A.list_i.ensure((size_t)groups * 8 * c->max_tris);
             A.list_f.ensure((size_t)groups * 12 * c->max_tris);
         }
@@ -1226,9 +1238,16 @@ void contact_pairs_impl(zdx_ctx* c, zdx_ctx::Api& A, const zdx_pair_in* pairs, i
         for (int attempt = 0; attempt < 10; ++attempt) {
             c->api_attempts = attempt + 1;
             A.arena.ensure((size_t)A.hit_cap * 6);
-            A.hits.ensure((c->clusters ? 8 : 6) * (size_t)A.hit_cap);
             A.hit_flag.ensure((size_t)A.hit_cap);
-            if (c->clusters) A.seg_tmp.ensure(6 * (size_t)A.hit_cap);
+            // the cluster path's hits and unsorted segments lie in the topology's
+            // buffers, its work items in the loop records (walk D's): each is
+            // done with before those are written
+            if (c->clusters) {
+                A.tw.ensure_narrow(A.hit_cap);
+                A.rec.ensure(std::max((size_t)n * A.lmax * 28, (size_t)n * sizeof(PairItem) / sizeof(double)));
+            } else {
+                A.hits.ensure(6 * (size_t)A.hit_cap);
+            }
             const bool sens = opts->sensitivities != 0;
             NarrowCfg nc{API_GROUP, 4, groups, batched ? 1 : 0, std::min(persistent_groups(c, 4), (n + 3) / 4)};
             nc.side = c->stream3; nc.ev_fork = c->ev_fork3; nc.ev_join = c->ev_join3;
@@ -1238,12 +1257,12 @@ void contact_pairs_impl(zdx_ctx* c, zdx_ctx::Api& A, const zdx_pair_in* pairs, i
             DPairs P{};
             P.cap = n; P.n = A.npairs.p; P.pi = A.pi.p; P.pj = A.pj.p; P.order = ordered ? A.order.p : nullptr;
             P.items = ordered ? A.items.p : nullptr;
-            P.pitems = A.pitems.p; P.seg_tmp = A.seg_tmp.p;
+            if (c->clusters) { P.pitems = (PairItem*)A.rec.p; P.seg_tmp = A.tw.seg_tmp(); }
             P.seg_off = A.seg_off.p; P.nseg = A.nseg.p; P.tri_checks = A.tri_checks.p; P.tri_tests = A.tri_tests.p;
             P.tri_hits = A.tri_hits.p; P.tri_scanned = A.tri_scanned.p; P.arena = A.arena.p; P.arena_cap = A.hit_cap;
             P.status = A.status.p;
             P.topo_list = A.topo_list.p; P.topo_n = A.topo_n.p;
-            P.hits = A.hits.p; P.hit_cap = A.hit_cap; P.hit_top = A.hit_top.p; P.hit_off = A.hit_off.p;
+            P.hits = c->clusters ? A.tw.hits() : A.hits.p; P.hit_cap = A.hit_cap; P.hit_top = A.hit_top.p; P.hit_off = A.hit_off.p;
             P.hit_shards = (int32_t)std::min<int64_t>(std::min<int64_t>(HIT_SHARDS, n), A.hit_cap);
             P.hit_flag = A.hit_flag.p;
             P.heavy = A.heavy.p;
@@ -1273,7 +1292,7 @@ void contact_pairs_impl(zdx_ctx* c, zdx_ctx::Api& A, const zdx_pair_in* pairs, i
             };
             // before the topology's buffers grow, whether the narrow phase's
             // were large enough for them to be sized
-            if (!lim.may_allocate || A.tw.cell9.n < 9 * (size_t)A.hit_cap ||
+            if (!lim.may_allocate || !A.tw.arena_holds(A.hit_cap) ||
                 (sens && A.vj.n < 72 * (size_t)A.hit_cap)) {
                 HIPC(hipMemcpyAsync(&head->status, A.status.p, 4, hipMemcpyDeviceToHost, st));
                 HIPC(hipMemcpyAsync(head->clock, A.stamps.p, 16, hipMemcpyDeviceToHost, st));
@@ -1992,7 +2011,7 @@ zdx_status zdx_sim_autotune(zdx_sim* s, int32_t* out_block, int32_t* out_groups)
     return guard(s->ctx, [&] {
         hipStream_t st = s->st();
         const int par = s->parity;
-        s->ensure_hits();
+        s->ensure_narrow();
         DBodies B = s->bodies(par);
         DMeshes M = s->ctx->dmeshes();
         launch_fill_i32(s->d_status.p, 0, 1, st);
