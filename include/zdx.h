@@ -272,11 +272,13 @@ zdx_status zdx_sim_set_force_model(zdx_sim* sim, int32_t model, double k);
  * tests: one of 6404, 6408, 12804, 12808, 25601, 25602, 25604, 25608, 51202,
  * 51204 (the compiled kernels); any other value returns ZDX_BAD_ARG.
  * np_groups_per_cu (1..16) sets its persistent grid to that many workgroups
- * per CU.  0 keeps the current value of either.  The autotuner
- * (zdx_sim_autotune) times every compiled shape, and the most float-box
- * tests a pair may have on the one-wave kernel (4096 or 16384), on the
- * current step's pair set and keeps the fastest; it reports the shape in the
- * same encoding. */
+ * per CU.  0 keeps the current value of either.  The tests per thread matter
+ * only where a registered mesh exceeds 65535 triangles or 65536 vertices (the
+ * kernels of all other contexts have none).  The autotuner (zdx_sim_autotune)
+ * times every compiled shape, and limits of the float-box tests a pair may
+ * have on the one-wave kernel, on the current step's pair set and keeps the
+ * fastest (the current one unless another is 2 % faster); it reports the shape
+ * in the same encoding. */
 zdx_status zdx_sim_set_tiles(zdx_sim* sim, int32_t np_shape, int32_t np_groups_per_cu);
 zdx_status zdx_sim_autotune(zdx_sim* sim, int32_t* np_shape, int32_t* np_groups_per_cu);
 

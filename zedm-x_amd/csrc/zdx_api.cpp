@@ -749,6 +749,9 @@ struct zdx_sim {
         tw.scr_i.release(); tw.scr_d.release();
         tw.ensure_slices(topo_threads, seg_max);
     }
+    // the pairs that bodies of like size can have (8 each, as the first pair
+    // buffers hold)
+    int64_t likely_pairs() const { return std::min<int64_t>((int64_t)N * (N - 1) / 2, 8 * (int64_t)N); }
     int32_t transform_groups() const { return std::max(1, ctx->n_cu * 8); }
 };
 
@@ -969,9 +972,8 @@ void enqueue_step(zdx_sim* s, int par, bool batched) {
     nc.groups = g_narrow;
     nc.wave_groups = persistent_groups(s->ctx, 4);
     nc.side = s->ctx->stream3; nc.ev_fork = s->ctx->ev_fork3; nc.ev_join = s->ctx->ev_join3;
-    // the pairs that bodies of like size can have (8 each, as the first
-    // pair buffers hold); plain mode has just read their number
-    nc.few = (batched ? std::min<int64_t>((int64_t)s->N * (s->N - 1) / 2, 8 * (int64_t)s->N) : n_pairs) <= PAIRS_FEW;
+    // plain mode has just read the number of pairs
+    nc.few = (batched ? s->likely_pairs() : n_pairs) <= PAIRS_FEW;
     if (nc.few) {
         nc.groups = (int)std::min<int64_t>(nc.groups, PAIRS_FEW);
         // one launch per topology stage, and two walks per CU at most: no big
@@ -2005,12 +2007,25 @@ zdx_status zdx_sim_set_tiles(zdx_sim* s, int32_t shape, int32_t groups_per_cu) {
 // Autotuner: times the narrow phase alone on the current step's pair set for
 // each (threads per workgroup, tests per thread, workgroups per CU of the
 // workgroup kernel; most tests of a pair on the one-wave kernel) and keeps the
-// fastest.  Every configuration produces the identical segment lists.
+// fastest.  Every configuration produces the identical segment lists.  The
+// cluster path has no tests per thread, so each workgroup size is timed once,
+// and the current configuration is timed first and kept unless another is 2 %
+// faster (what two timings of one differ by).  A simulation whose batched steps
+// give every pair a workgroup at once uses none of this and keeps its own.
 zdx_status zdx_sim_autotune(zdx_sim* s, int32_t* out_block, int32_t* out_groups) {
     if (!s) return ZDX_BAD_ARG;
     return guard(s->ctx, [&] {
         hipStream_t st = s->st();
         const int par = s->parity;
+        const bool clus = s->ctx->clusters;
+        auto report = [&] {
+            if (out_block) *out_block = s->ncfg.block * 100 + s->ncfg.items;
+            if (out_groups) *out_groups = s->np_groups_per_cu;
+        };
+        if (clus && s->likely_pairs() <= PAIRS_FEW) {
+            report();
+            return;
+        }
         s->ensure_narrow();
         DBodies B = s->bodies(par);
         DMeshes M = s->ctx->dmeshes();
@@ -2028,47 +2043,52 @@ zdx_status zdx_sim_autotune(zdx_sim* s, int32_t* out_block, int32_t* out_groups)
         DPairs P = s->dpairs(par, true);
         P.topo_big = P.topo_small = P.n_big = P.n_small = nullptr;   // timing the narrow phase only
         launch_lpt_order(P, M, B, s->d_order.p, s->d_bcnt.p, s->d_bcur.p, s->pair_cap, st);
-        const int cand[][2] = {{64, 4}, {64, 8}, {128, 4}, {128, 8}, {256, 1}, {256, 2}, {256, 4}, {256, 8},
-                               {512, 2}, {512, 4}};
+        struct Shape { int32_t block, items, groups, tests; };   // groups per CU; tests 0: the kernel's own limit
         const int gpc[] = {4, 8, 16};
+        std::vector<Shape> cand;
+        if (clus) {
+            cand.push_back({s->ncfg.block, s->ncfg.items, s->np_groups_per_cu, s->ncfg.wave_tests});
+            for (int bs : {64, 128, 256, 512})
+                for (int g : gpc)
+                    for (int wt : {4096, 16384, 0}) cand.push_back({bs, 4, g, wt});
+        } else {
+            const int cb[][2] = {{64, 4}, {64, 8}, {128, 4}, {128, 8}, {256, 1}, {256, 2}, {256, 4}, {256, 8},
+                                 {512, 2}, {512, 4}};
+            for (auto& c : cb)
+                for (int g : gpc)
+                    for (int wt : {4096, 16384}) cand.push_back({c[0], c[1], g, wt});
+        }
         hipEvent_t e0, e1;
         HIPC(hipEventCreate(&e0));
         HIPC(hipEventCreate(&e1));
         float best = 1e30f;
-        NarrowCfg bestc = s->ncfg;
-        int bestg = s->np_groups_per_cu;
-        // and the most float-box tests of a pair on the one-wave kernel
-        const int wtests[] = {4096, 16384};
-        for (auto& cb : cand) {
-            for (int g : gpc) for (int wt : wtests) {
-                NarrowCfg nc{cb[0], cb[1], persistent_groups(s->ctx, g), 1, persistent_groups(s->ctx, 4), wt};
-                nc.side = s->ctx->stream3; nc.ev_fork = s->ctx->ev_fork3; nc.ev_join = s->ctx->ev_join3;
-                // one untimed launch, then the median of four timed ones
-                float t4[4] = {0, 0, 0, 0};
-                for (int rep = 0; rep < 5; ++rep) {
-                    launch_fill_i32(s->d_topo_n.p, 0, 1, st);
-                    HIPC(hipEventRecord(e0, st));
-                    launch_narrow(B, M, P, nc, s->d_list_i.p, s->d_list_f.p, s->stage_cap, s->tmax,
-                                  s->d_queue.p, st);
-                    HIPC(hipEventRecord(e1, st));
-                    HIPC(hipEventSynchronize(e1));
-                    float ms = 0;
-                    HIPC(hipEventElapsedTime(&ms, e0, e1));
-                    if (rep > 0) t4[rep - 1] = ms;
-                }
-                std::sort(t4, t4 + 4);
-                const float tot = 0.5f * (t4[1] + t4[2]);
-                if (tot < best) { best = tot; bestc = nc; bestg = g; }
+        Shape bestc = cand[0];
+        for (const Shape& c : cand) {
+            NarrowCfg nc{c.block, c.items, persistent_groups(s->ctx, c.groups), 1, persistent_groups(s->ctx, 4), c.tests};
+            nc.side = s->ctx->stream3; nc.ev_fork = s->ctx->ev_fork3; nc.ev_join = s->ctx->ev_join3;
+            // one untimed launch, then the median of four timed ones
+            float t4[4] = {0, 0, 0, 0};
+            for (int rep = 0; rep < 5; ++rep) {
+                launch_fill_i32(s->d_topo_n.p, 0, 1, st);
+                HIPC(hipEventRecord(e0, st));
+                launch_narrow(B, M, P, nc, s->d_list_i.p, s->d_list_f.p, s->stage_cap, s->tmax, s->d_queue.p, st);
+                HIPC(hipEventRecord(e1, st));
+                HIPC(hipEventSynchronize(e1));
+                float ms = 0;
+                HIPC(hipEventElapsedTime(&ms, e0, e1));
+                if (rep > 0) t4[rep - 1] = ms;
             }
+            std::sort(t4, t4 + 4);
+            const float tot = 0.5f * (t4[1] + t4[2]);
+            if (tot < best) { best = &c == &cand[0] && clus ? 0.98f * tot : tot; bestc = c; }
         }
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
         s->ncfg.block = bestc.block;
         s->ncfg.items = bestc.items;
-        s->ncfg.wave_tests = bestc.wave_tests;
-        s->np_groups_per_cu = bestg;
-        if (out_block) *out_block = bestc.block * 100 + bestc.items;
-        if (out_groups) *out_groups = bestg;
+        s->ncfg.wave_tests = bestc.tests;
+        s->np_groups_per_cu = bestc.groups;
+        report();
     });
 }
 
