@@ -1,6 +1,8 @@
 // pass_a_large_emu.cpp — k_tp_pass_a on pairs whose endpoint pairs are past 32
 // bits of a product or of a count (23171 segments, 32769 segments): the first,
-// the middle and the last unit, against the serial tests of zdx_topo.h.
+// the middle and the last unit, against the serial tests of zdx_topo.h.  And the
+// larger pairs of a step in workgroups of PA_BIG_THREADS: the rows and words of
+// PA_THREADS, which pass_a_emu.cpp checks.
 #define main pass_a_emu_main
 #include "pass_a_emu.cpp"
 #undef main
@@ -81,8 +83,60 @@ static bool check_large(int S) {
     return nsnap > 4;
 }
 
+// adjacency counts and rows (slots past a row's count as they were) and snap
+// words of the larger pairs
+template <int NT>
+static std::vector<uint64_t> big_pairs(const Pairs& q, int groups) {
+    const int n = (int)q.S.size(), R = 6;
+    std::vector<int32_t> pi(n), nseg(q.S.begin(), q.S.end()), list(n), big, mesh(n), units;
+    std::vector<int64_t> seg_off = q.off, adj_off(n), snap_off(n);
+    std::vector<double> arena = q.arena, tol = q.tol;
+    int64_t na = 0, nw = 0;
+    for (int it = 0; it < n; ++it) {
+        const int S = nseg[it];
+        pi[it] = mesh[it] = list[it] = it;
+        adj_off[it] = na; snap_off[it] = nw;
+        na += (int64_t)S * (R + 1);
+        nw += ((int64_t)S * (2 * S - 1) + 63) / 64;
+        for (int b = 1; b < tp_pa_units(S); ++b) { units.push_back(it); units.push_back(b); }
+        if (S >= TOPO_BIG_SEGS) big.push_back(it);
+    }
+    std::vector<int32_t> adj(na, -7), cell9(9 * arena.size() / 6);
+    std::vector<uint64_t> snap(nw, 0x5555ull);
+    unsigned long long top[5] = {0, 0, 0, 0, units.size() / 2};
+    int32_t nn = n, nbig = (int)big.size(), none = 0;
+    TopoBufs T{cell9.data(), adj.data(), R, snap.data(), top, units.data(), (int64_t)units.size() / 2, adj_off.data(),
+               snap_off.data(), 0.02};
+    DPairs P{};
+    P.pi = pi.data(); P.nseg = nseg.data(); P.seg_off = seg_off.data(); P.arena = arena.data();
+    P.topo_list = list.data(); P.topo_n = &nn; P.topo_big = big.data(); P.n_big = &nbig; P.n_small = &none;
+    DMeshes M{};
+    M.tol = tol.data();
+    DBodies B{};
+    B.mesh = mesh.data();
+    const std::string err = simt::launch((unsigned)groups, NT, (size_t)pass_a_lds_bytes(NT, PA_WORDS, PA_SEGS),
+                                         [&] { k_tp_pass_a<NT, PA_WORDS, 2>(P, M, B, T, PA_SEGS); });
+    if (!err.empty()) {
+        std::printf("FAIL %s\n", err.c_str());
+        return {};
+    }
+    std::vector<uint64_t> out(snap);
+    for (int32_t a : adj) out.push_back((uint64_t)(int64_t)a);
+    out.push_back(top[3]);
+    return out;
+}
+static bool check_big() {
+    Pairs q = make_pairs();
+    for (double& x : q.arena)
+        if (!std::isfinite(x)) x = 0.25;   // the cells of others wrap
+    const std::vector<uint64_t> a = big_pairs<PA_THREADS>(q, 2), b = big_pairs<PA_BIG_THREADS>(q, 3);
+    const bool same = !a.empty() && a == b;
+    std::printf("%s %d threads as %d: %zu words\n", same ? "ok" : "FAIL", PA_BIG_THREADS, PA_THREADS, a.size());
+    return same;
+}
+
 int main() {
-    const bool ok = check_large(23300) && check_large(32900);
+    const bool ok = check_big() && check_large(23300) && check_large(32900);
     std::printf(ok ? "pass_a_large ok\n" : "pass_a_large failed\n");
     return ok ? 0 : 1;
 }

@@ -1,6 +1,7 @@
 """CPU: pass A's pair numbers where 32 bits end (tests/csrc/pass_a_large_emu.cpp):
 pairs of 23300 and 32900 segments, whose endpoint pairs number up to 2.2e9, under
-the SIMT emulation with signed overflow trapped."""
+the SIMT emulation with signed overflow trapped.  And the larger workgroups of a
+step's larger pairs, which give the rows and words of the smaller."""
 import os
 import shutil
 import subprocess

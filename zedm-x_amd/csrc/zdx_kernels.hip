@@ -2501,8 +2501,9 @@ static void launch_pass_a_small(const DPairs& P, const DMeshes& M, const DBodies
 // ... and of the others with their extra units (MODE 2), or of all (MODE 0)
 template <int MODE>
 static void launch_pass_a_big(const DPairs& P, const DMeshes& M, const DBodies& B, const TopoBufs& T, hipStream_t s) {
-    hipLaunchKernelGGL((k_tp_pass_a<PA_THREADS, PA_WORDS, MODE>), dim3((unsigned)T.pass_groups), dim3(PA_THREADS),
-                       (size_t)pass_a_lds_bytes(PA_THREADS, PA_WORDS, PA_SEGS), s, P, M, B, T, (int32_t)PA_SEGS);
+    constexpr int NT = MODE == 2 ? PA_BIG_THREADS : PA_THREADS;
+    hipLaunchKernelGGL((k_tp_pass_a<NT, PA_WORDS, MODE>), dim3((unsigned)T.pass_groups), dim3(NT),
+                       (size_t)pass_a_lds_bytes(NT, PA_WORDS, PA_SEGS), s, P, M, B, T, (int32_t)PA_SEGS);
 }
 static void launch_pass_a(const DPairs& P, const DMeshes& M, const DBodies& B, const TopoBufs& T, hipStream_t s,
                           bool zeroed = false, hipStream_t side = nullptr, hipEvent_t ev_fork = nullptr,

@@ -17,8 +17,10 @@
 // about 80 segments: 660 us with every pair taking the full tests (into an LDS
 // matrix of keys that one thread per row compacted, in 1024-thread workgroups),
 // 190 us so.  The pairs of the 100k bed (1900 small ones, 200 of 40 to 160
-// segments beside them): 37 and 51 us before, 31 and 55 so; one wave per small
-// pair 47, units of 16384 tests 95.
+// segments beside them, whose walks wait for it): 39 and 50 us before, 30 and
+// 32 so, the larger pairs in workgroups of 1024 threads (of 256 they take 64 us,
+// of 512 36: their 300 units leave the chip idle otherwise); one wave per small
+// pair 47.
 
 // Snap / adjacency tolerance of a pair: mesh A's (main.cpp:2118-2121) unless
 // the caller of the per-pair API gave one.
@@ -30,6 +32,7 @@ constexpr int PA_THREADS = 256;       // threads per unit of the larger pairs
 constexpr int PA_SEGS = 256;          // segments staged in LDS; a larger pair is read from memory
 constexpr int PA_WORDS = 512;         // snap words a unit builds in LDS at a time
 constexpr int PA_TESTS = 8192;        // segment-pair tests per unit (sets the units of a big pair)
+constexpr int PA_BIG_THREADS = 1024;  // where those are the few larger pairs of a step
 constexpr int PA_SMALL_THREADS = 128; // threads per pair of fewer than TOPO_BIG_SEGS segments
 constexpr int PA_SMALL_WORDS = 64;    // snap words of a pair of fewer than TOPO_BIG_SEGS segments
 static_assert((TOPO_BIG_SEGS - 1) * (2 * TOPO_BIG_SEGS - 3) <= 64 * PA_SMALL_WORDS, "a small pair's words");
