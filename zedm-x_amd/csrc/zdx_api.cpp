@@ -1080,8 +1080,7 @@ bool grow_for(zdx_sim* s, int32_t status, int par) {
 
 // Waits for the step's report: spins on rep->seq (set by the step's last
 // kernel).  The stream is asked whether it failed or drained only when a step
-// takes milliseconds, so hardly ever while one runs normally (asked every 256
-// spins, 100 steps of five bodies took 12.3 ms instead of 10.4).
+// takes milliseconds, so hardly ever while one runs normally.
 void wait_report(zdx_sim* s) {
     volatile unsigned int* seq = &s->rep->seq;
     for (uint64_t spin = 1;; ++spin) {
@@ -1113,7 +1112,7 @@ void step_once(zdx_sim* s, bool batched) {
         // The batched step too is launched kernel by kernel, not replayed from
         // a captured graph: host segmentation faults came up in replayed runs,
         // and their cause was not found.  Replay took 0.774 ms a step of the
-        // 100k bed and 0.101 of five bodies, this 0.793 and 0.104.
+        // 100k bed and 0.101 of five bodies, this 0.793 and 0.104 to 0.129.
         enqueue_step(s, par, batched);
         wait_report(s);
         const StepReport& r = *s->rep;

@@ -231,12 +231,18 @@ __device__ inline bool cluster_tri(const SideView& s, const CLoad& c, TriQ& q) {
     q.id = (uint16_t)(c.t >> 16);
     return (((unsigned)(w0 & w1 & w2) >> 16) == 0u) & ((c.t >> 16) != CLUS_NONE);
 }
-// outward-rounded float box of a kept triangle
+// outward-rounded float box of a kept triangle; a bound that is no number is
+// past every other, as the box test takes it, so that the boxes of groups hold it
 __device__ inline void kept_box(const double* wv, TriQ q, float* box) {
     V3 t[3] = {ld3(wv + 3 * (int)q.a), ld3(wv + 3 * (int)q.b), ld3(wv + 3 * (int)q.c)};
     double lo[3], hi[3];
     tri_box(t, lo, hi);
     box_f(lo, hi, box);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        box[k] = fmaxf(box[k], -INFINITY);
+        box[3 + k] = fminf(box[3 + k], INFINITY);
+    }
 }
 
 // boxes in LDS are read two floats at a time
