@@ -45,20 +45,24 @@ sys.path.insert(0, os.path.join(ROOT, "zedm-x_amd"))
 HBM_PEAK_GBS = 8000.0
 FP64_PEAK_TFLOPS = 78.6
 
-# algorithmic work of one narrow-phase launch (per step), from the counters:
-# FP64 ops: 24 per triangle scanned by the cull (3 corner loads, 12 min/max,
-#   6 compares, 6 outward roundings), 6 per executed AABB test, 200 per hit
-#   (exact AABB re-test 30, two planes 70, tri-tri 100), 100 per segment;
-# HBM bytes: 36 per triangle scanned (12 B of corner indices, 24 B of world
-#   vertex data: each vertex is shared by ~2 triangles) + 48 per segment written.
-OPS_PER_SCANNED, OPS_PER_TEST, OPS_PER_HIT, OPS_PER_SEG = 24, 6, 200, 100
-BYTES_PER_SCANNED, BYTES_PER_SEG = 36, 48
+# work of one step's narrow phase by clusters, from the counters, without what
+# no counter tells (the triangles of the clusters that meet, their boxes, the
+# triangle tests of groups that meet and hit nothing):
+# ops: 21 per cluster sphere, one for 15 of the bodies' triangles (tri_scanned);
+#   6 per test of two groups of 8 triangles (tri_tests is the product of the
+#   kept triangles); 200 per hit (exact AABB re-test 30, two planes 70, tri-tri
+#   100), 100 per segment;
+# HBM bytes: 16 per sphere; per hit its 32-byte record and six corners; per
+#   segment 48 written.
+OPS_PER_SCANNED, OPS_PER_TEST, OPS_PER_HIT, OPS_PER_SEG = 21 / 15, 6 / 64, 200, 100
+BYTES_PER_SCANNED, BYTES_PER_HIT, BYTES_PER_SEG = 16 / 15, 32 + 6 * 24, 48
 
 
 def narrow_model(ctr: dict):
     ops = (OPS_PER_SCANNED * ctr["tri_scanned"] + OPS_PER_TEST * ctr["tri_tests"] + OPS_PER_HIT * ctr["tri_hits"] +
            OPS_PER_SEG * ctr["segments"])
-    byts = BYTES_PER_SCANNED * ctr["tri_scanned"] + BYTES_PER_SEG * ctr["segments"]
+    byts = (BYTES_PER_SCANNED * ctr["tri_scanned"] + BYTES_PER_HIT * ctr["tri_hits"] +
+            BYTES_PER_SEG * ctr["segments"])
     return ops, byts
 
 
@@ -325,13 +329,22 @@ def _trace_by_kernel(d, pred):
     return {k: [t for _, t in sorted(v)] for k, v in rows.items()}
 
 
+def _steps_of(d, timed):
+    """Of each kernel's values in dispatch order, those of the last `timed` steps:
+    a kernel that a step launches twice has twice as many (the others, and so the
+    fewest, are launched once)."""
+    ref = min((len(v) for v in d.values()), default=1)
+    return {k: v[-timed * max(1, round(len(v) / ref)):] for k, v in d.items()}
+
+
 def _short(name):
     return name.replace("zdx::(anonymous namespace)::", "").split("(")[0].replace("void ", "")
 
 
-# the narrow phase (one launch each per step): clusters and box tests with one
-# wave per pair, then workgroups per pair for the two lists it leaves, exact
-# tests, ordering with the topology's work lists
+# the narrow phase: clusters and box tests with one wave per pair, then
+# workgroups per pair for the two lists it leaves (two launches, of one kernel
+# when both take 512 threads), exact tests, ordering with the topology's work
+# lists
 NARROW_KERNELS = ("k_pairs_",)
 NARROW_DESC = "narrow phase: k_pairs_wave + k_pairs_group (two lists, side by side) + k_pairs_exact + k_pairs_sort"
 
@@ -362,12 +375,12 @@ def summarize_profiles(stats_dir, fetch_dir, write_dir, command="", timed_stats=
     for r in stats[:30]:
         lines.append(f"| `{_short(r['Name'])}` | {r['Calls']} | {float(r['AverageNs']) / 1000:.1f} | "
                      f"{float(r['Percentage']):.2f} |")
-    tn = {k: v[-timed_stats:] for k, v in _trace_by_kernel(stats_dir, _is_narrow).items()}
+    tn = _steps_of(_trace_by_kernel(stats_dir, _is_narrow), timed_stats)
     if tn:
         lines += ["", f"Narrow phase over the last {timed_stats} steps (the timed steps), average per launch:"]
         for k, v in sorted(tn.items()):
             lines.append(f"- `{_short(k)}`: {sum(v) / len(v):.1f} us (min {min(v):.1f}, max {max(v):.1f})")
-        lines.append(f"- sum of these kernels: {sum(sum(v) / len(v) for v in tn.values()):.1f} us per step")
+        lines.append(f"- sum of these kernels' launches: {sum(sum(v) for v in tn.values()) / timed_stats:.1f} us per step")
     open(os.path.join(prof, "kernels_granular_bed_100k.md"), "w").write("\n".join(lines) + "\n")
     fetch = _pmc_by_kernel(fetch_dir, "FETCH_SIZE")
     write = _pmc_by_kernel(write_dir, "WRITE_SIZE")
@@ -379,9 +392,9 @@ def summarize_profiles(stats_dir, fetch_dir, write_dir, command="", timed_stats=
     is_copy = lambda k: ("copy" in k.lower() or "elementwise" in k.lower()) and "zdx" not in k
     cf, cw = pick(fetch, is_copy), pick(write, is_copy)
 
-    def per_step(d):   # mean per launch of each narrow kernel over the timed steps, summed
-        vals = {k: v[-timed_pmc:] for k, v in d.items() if _is_narrow(k)}
-        return sum(sum(v) / len(v) for v in vals.values()) if vals else 0.0, vals
+    def per_step(d):   # the narrow kernels' launches of a step, mean over the timed steps
+        vals = _steps_of({k: v for k, v in d.items() if _is_narrow(k)}, timed_pmc)
+        return sum(sum(v) for v in vals.values()) / timed_pmc, vals
 
     nf_kib, nf = per_step(fetch)
     nw_kib, nwr = per_step(write)
@@ -405,8 +418,8 @@ def summarize_profiles(stats_dir, fetch_dir, write_dir, command="", timed_stats=
         json.dump(res, open(os.path.join(prof, "narrow_traffic.json"), "w"), indent=1)
         md = ["# HBM traffic of the narrow phase -- granular bed, 100k polyhedra", "",
               f"Commands: `{command}` with `--pmc FETCH_SIZE` and `--pmc WRITE_SIZE` (separate runs)", "",
-              f"- kernels: {', '.join(_short(k) for k in sorted(nf))}, one launch each per step; the last "
-              f"{timed_pmc} steps (the timed steps)",
+              f"- kernels: {', '.join(_short(k) for k in sorted(nf))}, the last {timed_pmc} steps (the "
+              f"timed steps), means per launch",
               *[f"  - `{_short(k)}`: FETCH {sum(v) / len(v):.0f} KiB, WRITE {sum(nwr.get(k, [0])) / max(1, len(nwr.get(k, [0]))):.0f} KiB"
                 for k, v in sorted(nf.items())],
               f"- FETCH_SIZE per step: {nf_kib:.0f} KiB x scale {f_scale:.3f} = {fetch_b / 1e6:.1f} MB",

@@ -200,9 +200,9 @@ enum {
     ZDX_CTR_LOOPS = 4,
     ZDX_CTR_PAIRS = 5,        /* broad-phase candidate pairs (contact pairs evaluated) */
     ZDX_CTR_WALL_CONTACTS = 6,
-    ZDX_CTR_TRI_TESTS = 7,    /* triangle AABB tests actually executed after culling */
+    ZDX_CTR_TRI_TESTS = 7,    /* triangle pairs left by the culling (kept triangles of A times those of B) */
     ZDX_CTR_TRI_HITS = 8,     /* triangle pairs that reached the exact intersection test */
-    ZDX_CTR_TRI_SCANNED = 9,  /* triangles of both meshes scanned by the per-pair cull (sum of TA + TB) */
+    ZDX_CTR_TRI_SCANNED = 9,  /* triangles of both meshes of every pair (sum of TA + TB) */
     ZDX_CTR_TOPO_PAIRS = 10,  /* pairs with at least one intersection segment */
     ZDX_CTR_SEG_MAX = 11,     /* largest segment count of one pair (zdx_sim_stage_times: max over the steps) */
     ZDX_N_COUNTERS = 12
