@@ -24,8 +24,11 @@
 // Why: both of the kernels in zdx_narrow.h read every vertex and triangle of
 // both bodies and test the whole product of the kept triangles.  In the
 // 60k concave packing 5 % of the triangles are kept and 0.4 % of the product
-// hits; both passes were bound by instruction issue, and these still are, with
-// fewer instructions.  Narrow phase, those kernels / these, on an MI355X: 60k
+// hits, so most of that work is left out.  What bounds these: in the packing
+// instruction issue as far as its waves go (the vector units 51 % busy in the
+// wave kernel, 56 in the groups, 65 in the exact tests), in the 100k bed the
+// latency of a pair's chain (40, 22 and 51 %, 0.95 TB/s of memory traffic over
+// all four).  Narrow phase, those kernels / these, on an MI355X: 60k
 // packing 4241 / 1540 us, 4096 pairs of mixed meshes 1112 / 426, 257 pairs
 // with sensitivities 706 / 193, 100k bed 381 / 264.  (The exact test inside
 // the wave kernel, for its own hits, took 2760 us in the packing: partial
@@ -753,7 +756,8 @@ constexpr int TOPO_BIG_SEGS = 40;
 // (TOPO_BIG_SEGS or more) or topo_small.  4 to 256 pairs per workgroup, as the
 // grid needs: the lists take one atomic each per workgroup, then each wave
 // takes the next pair that has segments.  A pair with more than seg_cap stores
-// none (ST_STAGE).
+// none (ST_STAGE).  S^2/64 steps of one wave a pair: 26 us for the bed's 1900
+// pairs of up to 160 segments; a pair of 641 takes 0.29 ms of a call of 9.9.
 template <bool PROV>
 __global__ void __launch_bounds__(256) k_pairs_sort(DPairs P, int32_t seg_cap) {
     constexpr int NW = 256 / WAVE;

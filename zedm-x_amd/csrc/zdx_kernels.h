@@ -151,7 +151,12 @@ struct NarrowCfg {
     bool items_made = false;   // the work items are there (launch_pair_items), in pair order
 };
 // The most pairs that get a workgroup each at once: two workgroups of 512
-// threads fit on each of 256 CUs.
+// threads fit on each of 256 CUs.  A batched step, which does not know its
+// pairs, takes 8 a body for possible (zdx_sim::likely_pairs).  Both sides, us a
+// step, this route / the other: 64 bodies on a plane (106 pairs) 169 / 231; past
+// the line 256 bodies (477) 214 / 310, 1000 (1920) 307 / 321, 1500 (2882) 366 /
+// 337; beds of 500 to 2000 bodies (59 to 199) 220-265 / 306-359.  So the line is
+// on the safe side: the two are even near 2000 pairs.
 constexpr int64_t PAIRS_FEW = 512;
 // LDS of a topology walk then (two per CU).
 constexpr int32_t TOPO_LDS_FEW = 76 * 1024;
